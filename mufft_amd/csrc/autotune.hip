@@ -425,9 +425,9 @@ int mufft_hip_set_large_split(unsigned N, int kind, int code) {
 }
 
 // ===========================================================================
-// 2D column passes: the tile width of the column kernel (col_TX or its
-// alternative col_TX_alt) is chosen by timing both on the caller's image
-// shape.  The width changes only which columns a workgroup owns, so both
+// 2D column passes: the tile width of the column kernel (col_TX or an
+// alternative, col_TX_alt) is chosen by timing each on the caller's image
+// shape.  The width changes only which columns a workgroup owns, so all
 // must give identical bits; a width whose output differs is refused.
 // ===========================================================================
 static int mufft_hip_autotune_2d_impl(unsigned Nx, unsigned Ny, int kind, unsigned howmany, double *best_us) {
@@ -438,7 +438,6 @@ static int mufft_hip_autotune_2d_impl(unsigned Nx, unsigned Ny, int kind, unsign
         return -1;
     }
     const int ly = ilog2(Ny);
-    const int alt = col_TX_alt((int)Ny);
     const int dir = (tk == TK_C2C_FWD || tk == TK_R2C) ? -1 : 1;
     // Columns and row stride as the 2D plans lay them out (fft.c:664-792):
     // Nx complex columns per row, of which Nx/2 + 1 are transformed for r2c / c2r.
@@ -466,11 +465,11 @@ static int mufft_hip_autotune_2d_impl(unsigned Nx, unsigned Ny, int kind, unsign
         if (hipMemcpy(din.f2() + (size_t)b * img, h_in.data(), img * sizeof(float2), hipMemcpyHostToDevice) !=
             hipSuccess)
             rc = -1;
-    const int cands[2] = {col_TX((int)Ny), alt};
+    const int cands[1 + COL_TX_ALTS] = {col_TX((int)Ny), col_TX_alt((int)Ny, 0), col_TX_alt((int)Ny, 1)};
     std::vector<float2> first, h_out((size_t)img);
     int best = -1;
     double best_t = 1e30;
-    for (int ci = 0; ci < 2 && !rc; ++ci) {
+    for (int ci = 0; ci < 1 + COL_TX_ALTS && !rc; ++ci) {
         const int tx = cands[ci];
         if (tx <= 0) continue;
         Engine e;
@@ -542,7 +541,7 @@ int mufft_hip_get_column_tile(unsigned L) {
 
 int mufft_hip_set_column_tile(unsigned L, int tx) {
     if (!is_pow2(L) || L < 2 || ilog2(L) > COL_MAX_LOG2 ||
-        (tx != 0 && tx != col_TX((int)L) && tx != col_TX_alt((int)L))) {
+        (tx != 0 && !col_TX_valid((int)L, tx))) {
         set_err("unknown column length or tile width");
         return -1;
     }
@@ -599,7 +598,7 @@ static int mufft_hip_tune_load_impl(const char *path) {
             continue;
         }
         if (tk == TK_COLTILE) {
-            if (l < 1 || l > COL_MAX_LOG2 || (var != col_TX(1 << l) && var != col_TX_alt(1 << l))) continue;
+            if (l < 1 || l > COL_MAX_LOG2 || !col_TX_valid(1 << l, var)) continue;
             set_col_tx(l, var);
             record_tune(l, tk, var, us);
             ++n;

@@ -146,6 +146,20 @@ __device__ __forceinline__ void bstore_nt(__amdgpu_buffer_rsrc_t r, unsigned vof
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)voff, (int)soff, 2);
 }
 
+// Global access at a wave-uniform 64-bit row address plus a 32-bit byte
+// offset per lane; NT: streaming policy.
+template <bool NT>
+__device__ __forceinline__ float2 gload(const float2 *row, unsigned off) {
+    const u32x2 *p = reinterpret_cast<const u32x2 *>(reinterpret_cast<const char *>(row) + off);
+    return __builtin_bit_cast(float2, NT ? __builtin_nontemporal_load(p) : *p);
+}
+template <bool NT>
+__device__ __forceinline__ void gstore(float2 *row, unsigned off, float2 v) {
+    u32x2 *p = reinterpret_cast<u32x2 *>(reinterpret_cast<char *>(row) + off);
+    if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(u32x2, v), p);
+    else *p = __builtin_bit_cast(u32x2, v);
+}
+
 // Thread numbering for the c2r pre-pass resolve, which pairs bin k with bin
 // N - k.  When T >= 64 threads hold points lt + T*c, the owners of k and
 // N - k are threads lt and T - lt; numbering thread t as mirror_lt<T>(t)

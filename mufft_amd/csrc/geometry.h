@@ -162,36 +162,70 @@ MUFFT_HD constexpr int seq_first(int N, int R, int NP, bool rem_first) {
 // adjacent columns.  Lanes run along the columns (unit stride) so every row
 // segment of a tile is one coalesced access.
 // ---------------------------------------------------------------------------
-// Points per thread: all of a tiny column, 16 up to 4096 points, 32 beyond.
-MUFFT_HD constexpr int col_E(int L) { return L <= 16 ? L : (L <= 4096 ? 16 : 32); }
+// Points per thread: all of a tiny column, 16 up to 256 points, 32 beyond.
+// With 32, columns of 512 and 1024 points take two passes (32 x 16, 32 x 32)
+// instead of three, i.e. one LDS exchange instead of two; such a kernel holds
+// half the waves with twice the loads in flight each.
+MUFFT_HD constexpr int col_E(int L) { return L <= 16 ? L : (L <= 256 ? 16 : 32); }
 MUFFT_HD constexpr int col_T(int L) { return L / col_E(L); }
-// Tile width of the four-step column kernel (whose transposed store needs the
-// full complex tile in LDS).  Two columns from 4096 points on, so that two
-// tiles share a CU: 2^22 x 4 -7%, the same time at 2^22 x 16.
-MUFFT_HD constexpr int fs_TX(int L) {
-    return col_T(L) <= 32 ? 256 / col_T(L) : (col_T(L) <= 128 ? 8 : (L >= 4096 ? 2 : 4));
+// The plain column kernel, from sweeps on MI355X.  From L = 512 on it uses
+// the split LDS exchange (half the LDS of a tile) and from 1024 on split
+// twiddles; two 512-thread workgroups of a 67 KB tile share a CU at 1024 and
+// 2048 points.  The row segments of a tile should be whole 128-byte lines (16
+// columns), or neighbouring tiles fetch and write parts of the same lines;
+// the register file holds 16 columns of up to 1024 points twice per CU and 8
+// columns of 2048 points twice or of 4096 points once.  Against the former 16
+// points per thread (512: 8 columns; 2048, 4096: 4), whole 2D transforms, us:
+// c2c 512^2 x 64 124.9 -> 113.9, 1024^2 x 16 93.6 -> 87.9, 2048^2 x 4 112.3 ->
+// 97.9; real 4096^2 x 2 there and back 328 -> 303.  At 2048 points 4 columns
+// (110.5) and 16 columns in one workgroup per CU (108.2) lose to 8.
+MUFFT_HD constexpr int col_TX(int L) {
+    return L < 256 ? 256 / col_T(L) : (L <= 1024 ? 16 : (L <= 4096 ? 8 : 4));
 }
-MUFFT_HD constexpr int fs_WG(int L) { return col_T(L) * fs_TX(L); }
-// The plain column kernel, from sweeps on MI355X.  From L = 1024 on it uses
-// the split LDS exchange and split twiddles (half the LDS of a tile).  At
-// L = 1024 a 16-column tile (one 128-byte line per row) is 15% faster than 8
-// columns; at L = 2048 a 4-column tile (more, smaller workgroups per CU) is
-// 12% faster than 8; at L = 4096 the split exchange lets two 4-column tiles
-// share a CU (2D 4096^2: -5%); at L = 8192 it allows 4 columns instead of 2
-// (2D 8192^2: -6%, four-step 2^26: -19%).
-MUFFT_HD constexpr int col_TX(int L) { return L == 1024 ? 16 : (L == 2048 || L == 4096 || L == 8192 ? 4 : fs_TX(L)); }
-// The one alternative tile width compiled per column length (0: none): twice
-// the default below 1024 points, half or twice it from 1024 on where the LDS
-// and the 1024-thread workgroup allow.  The tile width changes only which
-// columns a workgroup owns, never the arithmetic, so every choice gives the
-// same bits; the 2D autotuner times both on the caller's image shape.
-MUFFT_HD constexpr int col_TX_alt(int L) {
-    return L < 128 ? 0 : (L <= 512 ? 2 * col_TX(L) : (L == 1024 ? 8 : (L == 2048 ? 8 : 2)));
+// Further tile widths compiled per column length (0: none).  The tile width
+// changes only which columns a workgroup owns, never the arithmetic, so every
+// choice gives the same bits; the 2D autotuner times them on the caller's
+// image shape.
+MUFFT_HD constexpr int col_TX_alt(int L, int i = 0) {
+    return i == 0 ? (L < 128 ? 0 : (L <= 256 ? 2 * col_TX(L) : (L <= 1024 ? 8 : (L == 2048 ? 4 : 2))))
+                  : (i == 1 && L == 4096 ? 4 : 0);
 }
-MUFFT_HD constexpr int col_xm(int L) { return L >= 1024 ? 1 : 0; }    // XMode
+constexpr int COL_TX_ALTS = 2;
+MUFFT_HD constexpr bool col_TX_valid(int L, int tx) {
+    return tx > 0 && (tx == col_TX(L) || tx == col_TX_alt(L, 0) || tx == col_TX_alt(L, 1));
+}
+MUFFT_HD constexpr int col_xm(int L) { return L >= 512 ? 1 : 0; }    // XMode
 MUFFT_HD constexpr int col_twm(int L) { return L >= 1024 ? 1 : 0; }   // TwMode
-MUFFT_HD constexpr int col_WG(int L) { return col_T(L) * col_TX(L); }
-MUFFT_HD constexpr int col_lds_rows(int L) { return L + L / col_E(L); }
+// Waves per SIMD to budget registers for (128 VGPRs at 4: the two workgroups
+// per CU that the LDS holds).
+MUFFT_HD constexpr int col_waves_per_simd(int L) { return L >= 512 ? 4 : 1; }
+
+// The four-step column kernel: points per thread, tile width, exchange and
+// twiddle modes.  It reads row segments of TX columns, whole 128-byte lines
+// up to 1024 points, and writes each column as one run; the split exchange
+// keeps two workgroups of 64-72 KB per CU from 1024 to 4096 points (one at
+// 8192).  Against 16 points per thread with a transposition through LDS in
+// full complex tiles half as wide, the first launch took, us per 512 MiB:
+// 265 -> 203 at 1024 points (2^20), 354 -> 265 at 4096 (2^22).
+MUFFT_HD constexpr int fs_E(int L) { return L <= 256 ? 16 : 32; }
+MUFFT_HD constexpr int fs_TX(int L) {
+    return L <= 64 ? 64 : (L == 128 ? 32 : (L <= 1024 ? 16 : (L == 2048 ? 8 : 4)));
+}
+MUFFT_HD constexpr int fs_WG(int L) { return L / fs_E(L) * fs_TX(L); }
+MUFFT_HD constexpr int fs_xm(int L) { return L >= 512 ? 1 : 0; }     // XMode
+MUFFT_HD constexpr int fs_twm(int L) { return L >= 512 ? 1 : 0; }    // TwMode
+MUFFT_HD constexpr int fs_waves_per_simd(int L) { return L >= 512 ? 4 : 1; }
+// LDS pitch of the columns of a tile of tx columns of `rows` slots (8 bytes
+// per slot, 4 in the split exchange): an odd multiple of u = (32 banks / words
+// per slot) / tx, so that tx columns times u consecutive slots, which the LDS
+// serves together, fall on different banks.
+MUFFT_HD constexpr int tile_pitch(int rows, int tx, int xm) {
+    const int banks = xm == 1 ? 32 : 16;
+    const int u = banks > tx ? banks / tx : 1;
+    const int q = (rows + u - 1) / u;
+    return (q % 2 ? q : q + 1) * u;
+}
+MUFFT_HD constexpr int fs_pitch(int L) { return tile_pitch(L + L / fs_E(L), fs_TX(L), fs_xm(L)); }
 constexpr int COL_MAX_LOG2 = 13;   // fused column kernel covers L <= 8192
 // Four-step split N = N1 * N2 for 2^17 <= N <= 2^26: log2 N1, the length of
 // the first launch's columns (the second launch's are N2 = N / N1).  From a

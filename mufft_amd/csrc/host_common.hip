@@ -248,7 +248,7 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         log_n2 = logn - log_n1;
         log_s = log_n2;
         const int n1 = 1 << log_n1, n2 = 1 << log_n2;
-        if (build_stockham_table(n1, dir, fused_sequence(n1, col_E(n1), false), &tw_fs1, s) ||
+        if (build_stockham_table(n1, dir, fused_sequence(n1, fs_E(n1), false), &tw_fs1, s) ||
             build_plain_table(n >> log_s, n >> log_s, dir, &tw_coarse, s) ||
             build_plain_table(n, 1 << log_s, dir, &tw_fine, s))
             return -1;

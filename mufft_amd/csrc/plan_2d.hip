@@ -86,9 +86,11 @@ static mufft_plan_2d *create_2d(int kind, unsigned Nx_c, unsigned Ny, int direct
     return guarded<mufft_plan_2d *>(nullptr, [&] { return create_2d_impl(kind, Nx_c, Ny, direction, flags); });
 }
 
+static size_t c2r_mid_stride(size_t Nx) { return Nx + 1; }
+
 size_t plan_2d_scratch_points(const mufft_plan_2d *p) {
     const size_t Nx = p->Nx, Ny = p->Ny;
-    if (p->kind == KIND_C2R) return (Nx + 1) * Ny;
+    if (p->kind == KIND_C2R) return c2r_mid_stride(Nx) * Ny;
     if (!p->ey.col_fused()) return (p->kind == KIND_C2C ? Nx : 2 * Nx) * Ny;
     return 0;
 }
@@ -117,7 +119,7 @@ static int exec_2d_images(mufft_plan_2d *p, void *out_, const void *in_, unsigne
     }
     // c2r: columns first (fft.c:863-916), then the per-row resolve and rows.
     const long long in_rs = 2 * Nx, in_img = in_rs * Ny;
-    const long long mid_rs = Nx + 1, mid_img = mid_rs * Ny;
+    const long long mid_rs = (long long)c2r_mid_stride(Nx), mid_img = mid_rs * Ny;
     if (s2.ensure(sizeof(float2) * (size_t)mid_img * hm)) return -1;
     if (run_cols(p->ey, in, in_rs, in_img, s2.f2(), mid_rs, mid_img, (int)(Nx + 1), hm, alt, st))
         return -1;

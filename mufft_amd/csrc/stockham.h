@@ -95,55 +95,48 @@ __device__ __forceinline__ void exchange_sync() {
     }
 }
 
-// v[c] holds point lt + T*c on entry (T = N/E) and holds output point lt + T*c
+// v[c] holds point lt + T*c on entry (T = N/E) and holds output point lt1 + T*c
 // on exit.  The passes follow seq_radix(): radix R (R <= E, default E) and
 // one remainder pass, first or last (REM_FIRST); each thread runs J = E/r
 // butterflies of a pass, butterfly j being b = lt + T*j over its points
 // v[j + m*J].  `twl` reads the twiddle table of that sequence.  `Slot(o)`
 // maps a point index to its LDS slot; `L` is the complex LDS view, `Lf` the
-// float view used by the split exchange.  The first pass may hold its points
-// under another thread numbering: with lt0 >= 0, v[c] holds point lt0 + T*c
-// on entry (lt0 a permutation of the threads); the first pass has no
-// twiddles and its results go through LDS, so the later passes and the
-// output use lt.
-template <int N, int E, int DIR, int XM, int TWM, int R = E, bool WAVE = false, bool REM_FIRST = true,
-          typename TwLoad, typename Slot>
-__device__ __forceinline__ void stockham_passes(float2 (&v)[E], int lt, TwLoad twl,
-                                                float2 *L, float *Lf, Slot slot, int lt0 = -1) {
+// float view used by the split exchange.
+// The thread numbering may change where points pass through LDS anyway:
+//  - the first pass runs under lt0 (v[c] holds point lt0 + T*c on entry; it
+//    has no twiddles);
+//  - the last exchange is read, and the last pass run, under lt1, through
+//    SlotR, the view of that exchange's LDS layout by the renumbered threads
+//    (SlotW is the writers' view).
+// stockham_passes() below keeps one numbering but for lt0.
+template <int N, int E, int DIR, int XM, int TWM, int R, bool WAVE, bool REM_FIRST, typename TwLoad,
+          typename Slot, typename SlotW, typename SlotR>
+__device__ __forceinline__ void stockham_passes_renumbered(float2 (&v)[E], int lt, TwLoad twl, float2 *L,
+                                                           float *Lf, Slot slot, int lt0, int lt1,
+                                                           SlotW slot_w, SlotR slot_r) {
     constexpr int T = N / E;
     constexpr int NP = np_for(N, R);
-    if (lt0 < 0) lt0 = lt;
     static_assert(R <= E && E % R == 0, "pass radix divides the points per thread");
     static_assert(!WAVE || T <= 64, "wave-local exchange needs the transform within one wave");
-    // Slot of point lt + T*c for the exchange reads.  The slot maps used here
-    // (padded: o + (o >> log2 E), scaled by a tile width and offset by a lane)
-    // split exactly over a multiple of E, so when E divides T every read is
-    // one per-thread base plus a compile-time offset; the compiler then keeps
-    // one address live instead of one per point, which it would otherwise
-    // hold (or spill) across all passes.
-    const int rd0 = slot(lt), rz = slot(0);
-    auto rd_slot = [&](auto C) {
-        constexpr int c = decltype(C)::value;
-        if constexpr (T % E == 0) return rd0 + (slot(T * c) - rz);
-        else return slot(lt + T * c);
-    };
     static_for<0, NP>([&](auto S) {
         constexpr int s = decltype(S)::value;
         constexpr int r = seq_radix(N, R, NP, s, REM_FIRST);
         constexpr int p = seq_p(N, R, NP, s, REM_FIRST);
         constexpr int J = E / r;   // butterflies per thread in this pass
+        const int ls = s == NP - 1 ? lt1 : lt;
         static_for<0, J>([&](auto JJ) {
             constexpr int j = decltype(JJ)::value;
             float2 u[r];
             static_for<0, r>([&](auto M) { u[decltype(M)::value] = v[j + decltype(M)::value * J]; });
             if constexpr (s > 0) {
-                const int k = (lt + T * j) & (p - 1);
+                const int k = (ls + T * j) & (p - 1);
                 apply_twiddles<r, p, TWM>(u, k, tw_offset(seq_first(N, R, NP, REM_FIRST), p), twl);
             }
             dft<r, DIR>(u);
             static_for<0, r>([&](auto Q) { v[j + decltype(Q)::value * J] = u[decltype(Q)::value]; });
         });
         if constexpr (s < NP - 1) {
+            constexpr bool LAST = s == NP - 2;
             // Output q of butterfly b goes to point (b - k)*r + k + q*p with
             // k = b mod p; the next pass reads points lt + T*c.
             auto publish = [&](auto get, auto put) {
@@ -154,27 +147,57 @@ __device__ __forceinline__ void stockham_passes(float2 (&v)[E], int lt, TwLoad t
                     const int base = (b - k) * r + k;
                     static_for<0, r>([&](auto Q) {
                         constexpr int q = decltype(Q)::value;
-                        put(slot(base + q * p), get(v[j + q * J]));
+                        if constexpr (LAST) put(slot_w(base + q * p), get(v[j + q * J]));
+                        else put(slot(base + q * p), get(v[j + q * J]));
                     });
                 });
+            };
+            // Slot of point lt + T*c for the reads.  The slot maps used here
+            // (padded: o + (o >> log2 E), scaled by a tile width and offset by
+            // a lane) split exactly into slot(lt) plus a constant when T and E
+            // divide one another, so every read is one per-thread base plus a
+            // compile-time offset; the compiler then keeps one address live
+            // instead of one per point, which it would otherwise hold (or
+            // spill) across all passes.
+            auto collect = [&](auto &sl, int base, auto take) {
+                const int rd0 = sl(base), rz = sl(0);
+                static_for<0, E>([&](auto C) {
+                    constexpr int c = decltype(C)::value;
+                    if constexpr (T % E == 0 || E % T == 0) take(C, rd0 + (sl(T * c) - rz));
+                    else take(C, sl(base + T * c));
+                });
+            };
+            auto collect_all = [&](auto take) {
+                if constexpr (LAST) collect(slot_r, lt1, take);
+                else collect(slot, lt, take);
             };
             if constexpr (XM != XM_SPLIT) {
                 publish([](float2 z) { return z; }, [&](int o, float2 z) { L[o] = z; });
                 exchange_sync<WAVE>();
-                static_for<0, E>([&](auto C) { v[decltype(C)::value] = L[rd_slot(C)]; });
+                collect_all([&](auto C, int o) { v[decltype(C)::value] = L[o]; });
                 exchange_sync<WAVE>();
             } else {
                 publish([](float2 z) { return z.x; }, [&](int o, float x) { Lf[o] = x; });
                 exchange_sync<WAVE>();
-                static_for<0, E>([&](auto C) { v[decltype(C)::value].x = Lf[rd_slot(C)]; });
+                collect_all([&](auto C, int o) { v[decltype(C)::value].x = Lf[o]; });
                 exchange_sync<WAVE>();
                 publish([](float2 z) { return z.y; }, [&](int o, float y) { Lf[o] = y; });
                 exchange_sync<WAVE>();
-                static_for<0, E>([&](auto C) { v[decltype(C)::value].y = Lf[rd_slot(C)]; });
+                collect_all([&](auto C, int o) { v[decltype(C)::value].y = Lf[o]; });
                 exchange_sync<WAVE>();
             }
         }
     });
+}
+
+// The passes under one thread numbering; with lt0 >= 0 the first pass runs
+// under lt0 (a permutation of the threads).
+template <int N, int E, int DIR, int XM, int TWM, int R = E, bool WAVE = false, bool REM_FIRST = true,
+          typename TwLoad, typename Slot>
+__device__ __forceinline__ void stockham_passes(float2 (&v)[E], int lt, TwLoad twl,
+                                                float2 *L, float *Lf, Slot slot, int lt0 = -1) {
+    stockham_passes_renumbered<N, E, DIR, XM, TWM, R, WAVE, REM_FIRST>(v, lt, twl, L, Lf, slot,
+                                                                        lt0 < 0 ? lt : lt0, lt, slot, slot);
 }
 
 }  // namespace mufft
