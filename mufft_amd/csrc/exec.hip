@@ -48,9 +48,13 @@ int run_generic(const Engine &e, const float2 *src, Lay s_lay, Lay fin, Lay alt,
 // c2c transforms beyond the fused row sizes, packed scratch `alt` of
 // batch * n points: four-step (two fused column launches, three for the
 // sizes of fs3_split) up to 2^(2 * COL_MAX_LOG2) points, generic passes
-// beyond.  src, dst and alt must be distinct.
+// beyond.  src, dst and alt must be distinct.  r2c_w / c2r_w: the resolve
+// table of a forward / inverse real transform whose resolve runs inside the
+// last / first launch (e.r2c_in_cols() / e.c2r_in_cols()); dst then holds, or
+// src is, the spectrum of n + 1 bins.
 int run_large(const Engine &e, const float2 *src, long long sd, float2 *dst, long long dd,
-              float2 *alt, int batch, bool zp, hipStream_t st) {
+              float2 *alt, int batch, bool zp, hipStream_t st, const float2 *r2c_w = nullptr,
+              const float2 *c2r_w = nullptr) {
     if (!e.four_step())
         return run_generic(e, src, Lay{const_cast<float2 *>(src), sd, 1}, Lay{dst, dd, 1},
                            Lay{alt, e.n, 1}, 1, batch, zp, st);
@@ -64,11 +68,37 @@ int run_large(const Engine &e, const float2 *src, long long sd, float2 *dst, lon
     f.in_bs = sd;
     f.out_bs = e.n;
     f.n2 = n2;
-    f.ntiles = n2 / fs_TX(n1);
     f.batch = batch;
     f.log2s = e.log_s;
     f.flags = zp ? RF_ZERO_PAD : 0u;
-    HIP_TRY(launch_four_step_cols(e.log_n1, e.direction, f, st));
+    if (c2r_w) {
+        RealFourStepArgs r{};
+        r.in = src;
+        r.out = alt;
+        r.tw = f.tw;
+        r.tw_self = e.tw_self;
+        r.coarse = f.coarse;
+        r.fine = f.fine;
+        r.rtw = c2r_w;
+        r.in_bs = sd;
+        r.out_bs = e.n;
+        r.n2 = n2;
+        r.batch = batch;
+        r.log2s = e.log_s;
+        HIP_TRY(launch_four_step_c2r(e.log_n1, r, st));
+    } else {
+        HIP_TRY(launch_four_step_cols(e.log_n1, e.direction, f, st));
+    }
+    RealColArgs rc{};
+    rc.in = alt;
+    rc.tw_self = e.tw_self;
+    rc.out = dst;
+    rc.rtw = r2c_w;
+    rc.in_bs = e.n;
+    rc.out_bs = dd;
+    rc.in_rs = n1;
+    rc.log_cols = e.log_n1;
+    rc.batch = batch;
     if (e.three_pass()) {
         // alt holds y[n2][k1], n2 = B*a + b.  Middle pass, in place: for each
         // (b, k1) the A-point transform over a (rows of B*N1 points), output
@@ -81,13 +111,20 @@ int run_large(const Engine &e, const float2 *src, long long sd, float2 *dst, lon
         c.in_rs = c.out_rs = (long long)nb * n1;
         c.in_bs = c.out_bs = e.n;
         c.ncols = nb * n1;
-        c.ntiles = (c.ncols + col_TX(na) - 1) / col_TX(na);
         c.batch = batch;
         c.coarse = e.tw_coarse2;
         c.fine = e.tw_fine2;
         c.log2s = e.log_s2;
         c.log2div = e.log_n1;
         HIP_TRY(launch_cols(e.log_a, e.direction, c, st, COL_TWIDDLE));
+        if (r2c_w) {
+            // The last pass below, column j = k1 + N1*k_a.
+            rc.tw = e.tw_pb;
+            rc.image_stride = (long long)nb * n1;
+            rc.m = na * n1;
+            HIP_TRY(launch_cols_r2c(e.log_b, rc, st));
+            return 0;
+        }
         // Last pass: for each (k_a, k1) the B-point transform over b; output
         // k_b is X[k1 + N1*(k_a + A*k_b)].  Image g = (transform, k_a).
         ColArgs d{};
@@ -102,12 +139,17 @@ int run_large(const Engine &e, const float2 *src, long long sd, float2 *dst, lon
         d.in_bs2 = e.n;
         d.out_bs2 = dd;
         d.ncols = n1;
-        d.ntiles = (n1 + col_TX(nb) - 1) / col_TX(nb);
         d.batch = batch * na;
         HIP_TRY(launch_cols(e.log_b, e.direction, d, st, COL_TWO_LEVEL));
         return 0;
     }
     // Second half: the N2-point column transforms of the n2 x n1 matrix.
+    if (r2c_w) {
+        rc.tw = e.tw_fs2;
+        rc.m = n1;
+        HIP_TRY(launch_cols_r2c(e.log_n2, rc, st));
+        return 0;
+    }
     ColArgs c{};
     c.in = alt;
     c.out = dst;
@@ -117,7 +159,6 @@ int run_large(const Engine &e, const float2 *src, long long sd, float2 *dst, lon
     c.in_bs = e.n;
     c.out_bs = dd;
     c.ncols = n1;
-    c.ntiles = (n1 + col_TX(n2) - 1) / col_TX(n2);
     c.batch = batch;
     // Columns of 64-1024 points (tile rows of whole cache lines) stream:
     // -3% to -7% at 2^17-2^22 points on MI355X.  With narrower tile rows
@@ -153,11 +194,18 @@ int run_rows(const Engine &e, int kind, const float2 *rtw, const float2 *in, lon
         HIP_TRY(launch_rows(e.logn, e.direction, kind, e.row_var, a, st));
         return 0;
     }
-    // Generic path: packed scratch of batch*n points each.
+    // Multi-launch paths: packed scratch of batch*n points each.
     const long long n = e.n;
     const size_t bytes = sizeof(float2) * (size_t)n * (size_t)batch;
-    if (s0.ensure(bytes) || s1.ensure(bytes)) return -1;
+    if (s1.ensure(bytes)) return -1;
     const bool zp = (flags & RF_ZERO_PAD) != 0;
+    // Plain real transforms resolve inside a column launch: 2^21 reals x 64,
+    // r2c 782 -> XXX us, c2r 797 -> XXX us.
+    if (kind == KIND_R2C && (flags & (RF_FULL | RF_ADJ_C2R)) == 0 && e.r2c_in_cols())
+        return run_large(e, in, idist, out, odist, s1.f2(), batch, zp, st, rtw);
+    if (kind == KIND_C2R && (flags & (RF_MUL | RF_ZERO_PAD | RF_ADJ_R2C)) == 0 && e.c2r_in_cols())
+        return run_large(e, in, idist, out, odist, s1.f2(), batch, false, st, nullptr, rtw);
+    if (s0.ensure(bytes)) return -1;
     if (kind == KIND_C2C) {
         const float2 *src = in;
         long long sd = idist;
@@ -230,9 +278,8 @@ int run_cols(const Engine &e, const float2 *src, long long rs_src, long long bs_
         a.out_rs = rs_dst;
         a.in_bs = bs_src;
         a.out_bs = bs_dst;
-        const int tx = e.col_tx ? e.col_tx : col_TX(e.n);
+        const int tx = e.col_tx ? e.col_tx : col_TX_for(e.n, ncols, batch);
         a.ncols = ncols;
-        a.ntiles = (ncols + tx - 1) / tx;
         a.batch = batch;
         HIP_TRY(launch_cols(e.logn, e.direction, a, st, COL_PLAIN, tx));
         return 0;

@@ -188,17 +188,28 @@ MUFFT_HD constexpr int col_TX(int L) {
 // image shape.
 MUFFT_HD constexpr int col_TX_alt(int L, int i = 0) {
     return i == 0 ? (L < 128 ? 0 : (L <= 256 ? 2 * col_TX(L) : (L <= 1024 ? 8 : (L == 2048 ? 4 : 2))))
-                  : (i == 1 && L == 4096 ? 4 : 0);
+                  : (i == 1 && L == 4096 ? 4 : 0);   // at 512-4096 points one is half the default
 }
 constexpr int COL_TX_ALTS = 2;
+// The width a plain launch over `images` of `ncols` columns takes: where full
+// tiles are at most 128, half the CUs, the half-width ones fill more of the
+// GPU (2D c2c, us: 1024 x 512 x 1 12.8 -> 11.9, 1024^2 x 1 17.0 -> 15.7, 512 x
+// 2048 x 1 20.3 -> 18.3; at 192 tiles of 2048 points 27.1 -> 30.6, so not
+// beyond).
+MUFFT_HD constexpr int col_TX_for(int L, int ncols, int images) {
+    return L >= 512 && L <= 4096 && (long long)((ncols + col_TX(L) - 1) / col_TX(L)) * images <= 128
+               ? col_TX(L) / 2 : col_TX(L);
+}
 MUFFT_HD constexpr bool col_TX_valid(int L, int tx) {
     return tx > 0 && (tx == col_TX(L) || tx == col_TX_alt(L, 0) || tx == col_TX_alt(L, 1));
 }
-MUFFT_HD constexpr int col_xm(int L) { return L >= 512 ? 1 : 0; }    // XMode
+// XMode: the split exchange, except in the narrower tiles, whose full complex
+// tile fits (half the barriers: a launch of few tiles waits for each).
+MUFFT_HD constexpr int col_xm(int L, int tx) { return L >= 512 && tx == col_TX(L) ? 1 : 0; }
 MUFFT_HD constexpr int col_twm(int L) { return L >= 1024 ? 1 : 0; }   // TwMode
 // Waves per SIMD to budget registers for (128 VGPRs at 4: the two workgroups
 // per CU that the LDS holds).
-MUFFT_HD constexpr int col_waves_per_simd(int L) { return L >= 512 ? 4 : 1; }
+MUFFT_HD constexpr int col_waves_per_simd(int L, int tx) { return L >= 512 && tx == col_TX(L) ? 4 : 1; }
 
 // The four-step column kernel: points per thread, tile width, exchange and
 // twiddle modes.  It reads row segments of TX columns, whole 128-byte lines
@@ -211,10 +222,19 @@ MUFFT_HD constexpr int fs_E(int L) { return L <= 256 ? 16 : 32; }
 MUFFT_HD constexpr int fs_TX(int L) {
     return L <= 64 ? 64 : (L == 128 ? 32 : (L <= 1024 ? 16 : (L == 2048 ? 8 : 4)));
 }
-MUFFT_HD constexpr int fs_WG(int L) { return L / fs_E(L) * fs_TX(L); }
-MUFFT_HD constexpr int fs_xm(int L) { return L >= 512 ? 1 : 0; }     // XMode
+MUFFT_HD constexpr int fs_xm(int L, int tx) { return L >= 512 && tx == fs_TX(L) ? 1 : 0; }     // XMode
 MUFFT_HD constexpr int fs_twm(int L) { return L >= 512 ? 1 : 0; }    // TwMode
-MUFFT_HD constexpr int fs_waves_per_simd(int L) { return L >= 512 ? 4 : 1; }
+MUFFT_HD constexpr int fs_waves_per_simd(int L, int tx) { return L >= 512 && tx == fs_TX(L) ? 4 : 1; }
+// Narrow tiles of the column launches of 1D transforms (the four-step's first
+// launch, the column kernel's other modes, the real transforms' launches), for
+// launches whose full tiles are at most 128, half the CUs; the same bits.
+// NARROW_FIGURES
+MUFFT_HD constexpr int narrow_TX(int L, int tx) {
+    return L < 256 || L > 4096 ? 0 : (L <= 1024 ? tx / 4 : tx / 2);
+}
+MUFFT_HD constexpr bool use_narrow(int L, int tx, long long ncols, long long images) {
+    return narrow_TX(L, tx) > 0 && (ncols + tx - 1) / tx * images <= 128;
+}
 // LDS pitch of the columns of a tile of tx columns of `rows` slots (8 bytes
 // per slot, 4 in the split exchange): an odd multiple of u = (32 banks / words
 // per slot) / tx, so that tx columns times u consecutive slots, which the LDS
@@ -225,7 +245,21 @@ MUFFT_HD constexpr int tile_pitch(int rows, int tx, int xm) {
     const int q = (rows + u - 1) / u;
     return (q % 2 ? q : q + 1) * u;
 }
-MUFFT_HD constexpr int fs_pitch(int L) { return tile_pitch(L + L / fs_E(L), fs_TX(L), fs_xm(L)); }
+MUFFT_HD constexpr int fs_pitch(int L, int tx) { return tile_pitch(L + L / fs_E(L), tx, fs_xm(L, tx)); }
+
+// The column launches of large real transforms with the resolve fused in
+// (real_cols.hip): each thread holds its points of two columns.
+MUFFT_HD constexpr int rc_TX(int L) { return L <= 64 ? 64 : (L == 128 ? 32 : 16); }
+MUFFT_HD constexpr int rc_xm(int L, int tx) { return L >= 512 && tx == rc_TX(L) ? 1 : 0; }     // XMode
+MUFFT_HD constexpr int rc_twm(int L) { return L >= 512 ? 1 : 0; }    // TwMode
+MUFFT_HD constexpr int rc_waves_per_simd(int L) { return L >= 512 ? 2 : 1; }
+// Self-paired columns: points per thread and threads of a column.
+MUFFT_HD constexpr int rcs_E(int L) { return 4; }
+MUFFT_HD constexpr int rcs_T(int L) { return L / rcs_E(L); }
+// Lengths of the launches the fused kernels cover: the last column launch of
+// a forward transform, the first one of an inverse transform.
+MUFFT_HD constexpr bool real_col_fused(int logL) { return logL >= 6 && logL <= 10; }
+MUFFT_HD constexpr bool real_four_step_fused(int logN1) { return logN1 >= 8 && logN1 <= 10; }
 constexpr int COL_MAX_LOG2 = 13;   // fused column kernel covers L <= 8192
 // Four-step split N = N1 * N2 for 2^17 <= N <= 2^26: log2 N1, the length of
 // the first launch's columns (the second launch's are N2 = N / N1).  From a

@@ -142,6 +142,7 @@ bool variant_is_set(int logn, int tk);
 int chosen_fs_code(int logn);
 void set_fs_code(int logn, int code);
 int chosen_col_tx(int logL);
+int set_col_tx_or_0(int logL);   // 0: not set, the static choice
 void set_col_tx(int logL, int tx);
 
 // ---- one transform axis ----------------------------------------------------
@@ -163,7 +164,8 @@ struct Engine {
     // the twiddle w_N2^(b*k_a) from its own two-level tables.
     int log_a = 0, log_b = 0, log_s2 = 0;
     int fs_code = 0;              // the split in use (fs_code_*)
-    int col_tx = 0;               // column tile width (0 = col_TX(n))
+    int col_tx = 0;               // column tile width (0 = col_TX_for(n, columns, images))
+    float2 *tw_self = nullptr;    // self-paired columns of a real transform (real_cols.hip)
     float2 *tw_pa = nullptr, *tw_pb = nullptr, *tw_coarse2 = nullptr, *tw_fine2 = nullptr;
     std::vector<int> gen_radix;
 
@@ -171,6 +173,15 @@ struct Engine {
     bool row_fused() const { return logn <= ROW_MAX_LOG2; }
     bool col_fused() const { return logn <= COL_MAX_LOG2; }
     bool four_step() const { return logn > ROW_MAX_LOG2 && logn <= 2 * COL_MAX_LOG2; }
+    // Whether the resolve of a real transform runs inside the last (r2c) or
+    // first (c2r) column launch (real_cols.hip), whose tiles must be whole.
+    bool r2c_in_cols() const {
+        const int l = three_pass() ? log_b : log_n2;
+        return four_step() && real_col_fused(l) && (1 << log_n1) % (2 * rc_TX(1 << l)) == 0;
+    }
+    bool c2r_in_cols() const {
+        return four_step() && real_four_step_fused(log_n1) && (1 << log_n2) % (2 * rc_TX(1 << log_n1)) == 0;
+    }
     int launches_generic() const { return (int)gen_radix.size(); }
 
     // rows / cols: which roles this engine serves; kind: KIND_* of the row

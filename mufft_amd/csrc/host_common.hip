@@ -211,9 +211,13 @@ void set_fs_code(int logn, int code) {
     if (logn >= 0 && logn <= 2 * COL_MAX_LOG2) g_fs_code[logn] = code;
 }
 
-int chosen_col_tx(int logL) {
+int set_col_tx_or_0(int logL) {
     std::lock_guard<std::mutex> g(g_var_lock);
-    const int t = (logL >= 0 && logL <= COL_MAX_LOG2) ? g_col_tx[logL] : 0;
+    return (logL >= 0 && logL <= COL_MAX_LOG2) ? g_col_tx[logL] : 0;
+}
+
+int chosen_col_tx(int logL) {
+    const int t = set_col_tx_or_0(logL);
     return t ? t : col_TX(1 << logL);
 }
 
@@ -234,7 +238,7 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         if (rv_split(row_var) > 0 && build_split_table(n, n2, dir, &tw_split, s)) return -1;
     }
     if (cols && col_fused()) {
-        col_tx = tx ? tx : chosen_col_tx(logn);
+        col_tx = tx ? tx : set_col_tx_or_0(logn);
         if (build_stockham_table(n, dir, fused_sequence(n, col_E(n), false), &tw_col, s)) return -1;
     }
     if (rows && four_step()) {
@@ -265,6 +269,10 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         } else if (build_stockham_table(n2, dir, fused_sequence(n2, col_E(n2), false), &tw_fs2, s)) {
             return -1;
         }
+        // The real transforms' self-paired columns: r2c in the last launch, c2r in the first.
+        const int ns = kind == KIND_R2C && r2c_in_cols() ? 1 << (f3 ? log_b : log_n2)
+                     : kind == KIND_C2R && c2r_in_cols() ? n1 : 0;
+        if (ns && build_stockham_table(ns, dir, fused_sequence(ns, rcs_E(ns), false), &tw_self, s)) return -1;
     }
     if ((rows && !row_fused() && !four_step()) || (cols && !col_fused())) {
         gen_radix = generic_sequence(n);
@@ -275,11 +283,11 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
 
 void Engine::release() {
     for (float2 *t : {tw_row, tw_col, tw_gen, tw_split, tw_fs1, tw_fs2, tw_coarse, tw_fine, tw_pa, tw_pb,
-                      tw_coarse2, tw_fine2})
+                      tw_coarse2, tw_fine2, tw_self})
         if (t) (void)hipFree(t);
     tw_row = tw_col = tw_gen = tw_split = nullptr;
     tw_fs1 = tw_fs2 = tw_coarse = tw_fine = nullptr;
-    tw_pa = tw_pb = tw_coarse2 = tw_fine2 = nullptr;
+    tw_pa = tw_pb = tw_coarse2 = tw_fine2 = tw_self = nullptr;
 }
 
 }  // namespace mufft

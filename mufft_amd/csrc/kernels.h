@@ -69,6 +69,37 @@ struct FourStepArgs {
     unsigned flags;        // RF_ZERO_PAD: rows n1 >= N1/2 are zero
 };
 
+// Last column launch of a forward real transform, resolve included: column
+// j < m of the n = m*L points, j >> log_cols its input image (image_stride
+// apart), rows in_rs apart; bin j + m*k2 of the spectrum at out + j + m*k2.
+struct RealColArgs {
+    const float2 *in;
+    float2 *out;
+    const float2 *tw;      // Stockham table of the L-point column kernel
+    const float2 *tw_self; // and of the self-paired columns' kernel
+    const float2 *rtw;     // resolve twiddles W[k], k < n
+    long long in_bs, out_bs;   // transform distance (complex elements)
+    long long in_rs, image_stride;
+    int log_cols;
+    int m;
+    int ntiles;            // tiles of the columns [0, m/2) per transform
+    int batch;
+};
+
+// First launch of an inverse real transform, resolve included: the spectrum
+// (n + 1 bins) as an N1 x n2 matrix; otherwise as FourStepArgs.
+struct RealFourStepArgs {
+    const float2 *in;
+    float2 *out;
+    const float2 *tw, *tw_self, *coarse, *fine;
+    const float2 *rtw;
+    long long in_bs, out_bs;
+    int n2;
+    int ntiles;            // tiles of the columns [0, n2/2) per transform
+    int batch;
+    int log2s;
+};
+
 // One Stockham pass of radix R over global memory (fallback for any size).
 struct PassArgs {
     const float2 *in;
@@ -129,7 +160,8 @@ hipError_t launch_rows(int logN, int direction, int kind, int var, const RowArgs
 // bits are left out (they run the same kernel for the other kinds).
 int row_variant_list(int logN, int *vars, int max, bool c2r = true);
 bool row_variant_registered(int logN, int var);
-// tx: tile width, col_TX(L) (0) or col_TX_alt(L) (plain mode only); ntiles must cover ncols.
+// tx: tile width in plain mode, col_TX(L) (0) or a col_TX_alt(L); the other
+// modes choose their own (0).  The launchers set ntiles.
 hipError_t launch_cols(int logL, int direction, const ColArgs &a, hipStream_t s, int mode = COL_PLAIN, int tx = 0);
 hipError_t launch_pass(int radix, int direction, const PassArgs &a, hipStream_t s);
 hipError_t launch_resolve_r2c(const ResolveArgs &a, hipStream_t s);
@@ -138,6 +170,9 @@ hipError_t launch_mul(const MulArgs &a, hipStream_t s);
 hipError_t launch_fold(const MulArgs &a, hipStream_t s);
 hipError_t launch_mul_reduce(const MulArgs &a, hipStream_t s);
 hipError_t launch_four_step_cols(int logN1, int direction, const FourStepArgs &a, hipStream_t s);
+// Each launches two kernels: the self-paired columns, then the pairs.
+hipError_t launch_cols_r2c(int logL, const RealColArgs &a, hipStream_t s);
+hipError_t launch_four_step_c2r(int logN1, const RealFourStepArgs &a, hipStream_t s);
 hipError_t launch_stream_copy(const float2 *in, float2 *out, long long n, hipStream_t s);
 hipError_t launch_ola(const float *y, float *out, const float *tail_in, float *tail_out,
                       long long n, long long nblocks, hipStream_t s);

@@ -86,7 +86,8 @@ static mufft_plan_2d *create_2d(int kind, unsigned Nx_c, unsigned Ny, int direct
     return guarded<mufft_plan_2d *>(nullptr, [&] { return create_2d_impl(kind, Nx_c, Ny, direction, flags); });
 }
 
-static size_t c2r_mid_stride(size_t Nx) { return Nx + 1; }
+// Row stride of the c2r intermediate image (Nx + 1 columns).
+static size_t c2r_mid_stride(size_t Nx) { return Nx >= 1024 ? Nx + 64 : Nx + 1; }
 
 size_t plan_2d_scratch_points(const mufft_plan_2d *p) {
     const size_t Nx = p->Nx, Ny = p->Ny;
