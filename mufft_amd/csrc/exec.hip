@@ -200,7 +200,7 @@ int run_rows(const Engine &e, int kind, const float2 *rtw, const float2 *in, lon
     if (s1.ensure(bytes)) return -1;
     const bool zp = (flags & RF_ZERO_PAD) != 0;
     // Plain real transforms resolve inside a column launch: 2^21 reals x 64,
-    // r2c 782 -> XXX us, c2r 797 -> XXX us.
+    // r2c 805 -> 564 us, c2r 796 -> 492 us (half of it from the column kernels).
     if (kind == KIND_R2C && (flags & (RF_FULL | RF_ADJ_C2R)) == 0 && e.r2c_in_cols())
         return run_large(e, in, idist, out, odist, s1.f2(), batch, zp, st, rtw);
     if (kind == KIND_C2R && (flags & (RF_MUL | RF_ZERO_PAD | RF_ADJ_R2C)) == 0 && e.c2r_in_cols())
