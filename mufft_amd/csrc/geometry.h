@@ -263,6 +263,28 @@ MUFFT_HD constexpr int rcs_T(int L) { return L / rcs_E(L); }
 // a forward transform, the first one of an inverse transform.
 MUFFT_HD constexpr bool real_col_fused(int logL) { return logL >= 6 && logL <= 10; }
 MUFFT_HD constexpr bool real_four_step_fused(int logN1) { return logN1 >= 8 && logN1 <= 10; }
+
+// Fused overlap-add (ola_fused.hip) on blocks of n complex points (N = 2n
+// reals): points per thread, threads per workgroup (at least two slots; 256
+// where that gives them: 512 took 12-30% longer) and slots.
+MUFFT_HD constexpr int ola_E(int n) { return n < 16 ? n : 16; }
+MUFFT_HD constexpr int ola_WG(int n) { return 2 * n / ola_E(n) > 256 ? 2 * n / ola_E(n) : 256; }
+MUFFT_HD constexpr int ola_slots(int n) { return ola_WG(n) / (n / ola_E(n)); }
+MUFFT_HD constexpr int ola_waves_per_simd(int n, bool many) { return n < 16 ? 1 : (many ? 3 : 4); }
+constexpr int OLA_MAX_LOG2 = 12;   // n; beyond, three launches (8192 points in one: 21.2 us for 8 blocks against 19.0)
+// Rounds of blocks a workgroup runs.  With two slots every other block of a
+// single round runs twice; at 2048 points (256 threads) more rounds pay once
+// the workgroups outnumber what the GPU holds (1024): N = 4096, us with one
+// round and with more: 2048 blocks 29.4 / 25.1, 16384 blocks 208 / 138.  With
+// more slots, and at 4096 points (two workgroups per CU instead of three once
+// the tail is kept in LDS), one round is as fast or faster: N = 2048 x 4096 21
+// / 29, N = 8192 x 2048 60 / 64.
+MUFFT_HD constexpr bool ola_rounds(int n) { return ola_slots(n) == 2 && ola_WG(n) == 256; }
+MUFFT_HD constexpr int ola_run(int n, long long nblocks) {
+    if (!ola_rounds(n) || nblocks <= 1024) return 1;
+    const long long r = (nblocks / 1536 + 3) / 2;
+    return r < 2 ? 2 : (r > 16 ? 16 : (int)r);
+}
 constexpr int COL_MAX_LOG2 = 13;   // fused column kernel covers L <= 8192
 // Four-step split N = N1 * N2 for 2^17 <= N <= 2^26: log2 N1, the length of
 // the first launch's columns (the second launch's are N2 = N / N1).  From a

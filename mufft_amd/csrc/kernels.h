@@ -100,6 +100,19 @@ struct RealFourStepArgs {
     int log2s;
 };
 
+// Overlap-add filtering in one launch (ola_fused.hip): nblocks blocks of n/2
+// complex points (two reals each) in and out.
+struct OlaArgs {
+    const float2 *in;
+    float2 *out;
+    const float2 *tw_fwd, *tw_inv;   // Stockham tables, remainder pass first
+    const float2 *ca, *cb;           // coefficients per bin k < n
+    const float2 *tail_in;           // n/2 points
+    float2 *tail_out;
+    long long nblocks;
+    int run;                         // blocks per slot (the launcher sets it)
+};
+
 // One Stockham pass of radix R over global memory (fallback for any size).
 struct PassArgs {
     const float2 *in;
@@ -174,6 +187,8 @@ hipError_t launch_four_step_cols(int logN1, int direction, const FourStepArgs &a
 hipError_t launch_cols_r2c(int logL, const RealColArgs &a, hipStream_t s);
 hipError_t launch_four_step_c2r(int logN1, const RealFourStepArgs &a, hipStream_t s);
 hipError_t launch_stream_copy(const float2 *in, float2 *out, long long n, hipStream_t s);
+hipError_t launch_ola_fused(int logn, const OlaArgs &a, hipStream_t s);
+hipError_t launch_ola_coeff(const float2 *H, float2 *ca, float2 *cb, int n, hipStream_t s);
 hipError_t launch_ola(const float *y, float *out, const float *tail_in, float *tail_out,
                       long long n, long long nblocks, hipStream_t s);
 hipError_t launch_twiddles(const TwiddleArgs &a, hipStream_t s);
