@@ -212,11 +212,11 @@ def conv_jobs_host():
 def conv_batch_bench(dev, stream, reps: int = 10):
     """Uneven convolution batch: 512 mono jobs, N = 2^(8 + u mod 9) real, signal
     N/2 uniform, filter N/2 taps z_n*exp(-n/(N/8)), z ~ N(0,1); plus 128 stereo
-    jobs N = 16384 (complex signal N/2).  One graph launch (one persistent
+    jobs N = 16384 (complex signal N/2).  One launch (one persistent
     kernel: forward then inverse tasks per job group, per-XCD queues) versus
     the per-plan drop-in path (plans cached per N, 3 synchronous calls per
     job) and the batched conv API (one batched call per (N, method) group and
-    step); the same kernel launched without the graph is reported too."""
+    step); the second entry point, the same launch, is reported too."""
     import torch
 
     import mufft_amd as M

@@ -94,6 +94,13 @@ int mufft_hip_execute_plan_1d_mul_batched(mufft_plan_1d *plan, void *output, con
                                           const void *input2, unsigned howmany, size_t idist,
                                           size_t idist2, size_t odist, float norm, int conj2,
                                           int adjoint, void *stream);
+/* The same, writing only the first half of each output (N/2 points or reals;
+ * odist 0 packs the halves): the gradient of a zero-padded input.  Up to 65536
+ * complex points. */
+int mufft_hip_execute_plan_1d_mul_head_batched(mufft_plan_1d *plan, void *output, const void *input,
+                                               const void *input2, unsigned howmany, size_t idist,
+                                               size_t idist2, size_t odist, float norm, int conj2,
+                                               int adjoint, void *stream);
 /* output[i] = norm * sum_b a_b[i] * op(b_b[i]), i < n (complex), op = conj when
  * conj_b != 0: the batch reduction of a filter gradient.  Deterministic. */
 int mufft_hip_mul_reduce(void *output, const void *a, const void *b, unsigned n, unsigned howmany,
@@ -158,10 +165,11 @@ int mufft_hip_get_large_split(unsigned N, int kind);
 /* code 0 restores the static split. */
 int mufft_hip_set_large_split(unsigned N, int kind, int code);
 /* 2D column passes: the fused column kernel of length Ny owns tiles of
- * adjacent columns; two tile widths are compiled per length from 128 points
- * on.  The autotuner times both on an Nx x Ny image batch of the given kind
+ * adjacent columns; two or three tile widths are compiled per length from 128
+ * points on, and each launch picks one where none is set.  The autotuner times
+ * them on an Nx x Ny image batch of the given kind
  * (real Nx for r2c / c2r, whose columns are Nx/2 + 1), requires identical
- * bits and selects the faster for plans created afterwards.  Returns the
+ * bits and selects the fastest for plans created afterwards.  Returns the
  * width.  The reference picks its vertical passes by a fixed rule
  * (fft.c:382-435). */
 int mufft_hip_autotune_2d(unsigned Nx, unsigned Ny, int kind, unsigned howmany, double *best_us);
@@ -175,7 +183,7 @@ int mufft_hip_tune_load(const char *path);
 
 /* ---- Uneven convolution batch ----
  * Many fast convolutions of mixed sizes and methods in one persistent kernel
- * launch fed by a device work queue, replayed from a captured hipGraph.  Each
+ * launch fed by a device work queue, which a caller may capture.  Each
  * job is one mufft_plan_conv round (both inputs transformed, multiplied,
  * inverse transformed, normalised by 1/N) on device buffers:
  *   first:  N/2 reals (mono) or N/2 complex (stereo) with the matching
@@ -200,9 +208,10 @@ typedef struct mufft_hip_conv_batch mufft_hip_conv_batch;
 
 mufft_hip_conv_batch *mufft_hip_create_conv_batch(const mufft_hip_conv_job *jobs, unsigned count,
                                                   unsigned flags);
-/* Replays the captured graph on stream (NULL: the batch's stream, and waits). */
+/* Launches the batch on stream (NULL: the batch's stream, and waits); on a
+ * capturing stream it becomes one kernel node of the caller's graph. */
 int mufft_hip_execute_conv_batch(mufft_hip_conv_batch *batch, void *stream);
-/* Same kernel without the graph. */
+/* The same. */
 int mufft_hip_execute_conv_batch_direct(mufft_hip_conv_batch *batch, void *stream);
 /* 0 = every execution so far ran every task, 1 = one did not (synchronises the device). */
 int mufft_hip_conv_batch_status(mufft_hip_conv_batch *batch);

@@ -163,8 +163,10 @@ class Plan1D:
         """The fused-kernel variant this plan runs (0: no fused row kernel)."""
         return int(_lib.load().mufft_hip_plan_1d_variant(self._h))
 
-    def _validate(self, out, inp, howmany, idist, odist, adjoint=False, inp2=None, idist2=0):
+    def _validate(self, out, inp, howmany, idist, odist, adjoint=False, inp2=None, idist2=0, head=False):
         ni, ei, no, eo = layout_1d(self.kind, self.N, self.flags, adjoint)
+        if head:
+            no //= 2
         if inp2 is not None and self.kind == "c2c":
             ni = self.N  # the fused multiply reads every input point, zero padding or not
         check_buffer(inp, span_bytes(howmany, idist, ni, ei), "input")
@@ -192,11 +194,14 @@ class Plan1D:
 
     def execute_mul_batched(self, out, inp, inp2, howmany: int, idist: int = 0, idist2: int = 0,
                             odist: int = 0, norm: float = 1.0, conj2: bool = False,
-                            adjoint: bool = False, stream=None):
+                            adjoint: bool = False, stream=None, head: bool = False):
         """out = T(norm * inp * op(inp2)) with the multiply fused into the transform;
-        idist2 = 0 applies one inp2 block to every transform."""
-        self._validate(out, inp, howmany, idist, odist, adjoint=adjoint, inp2=inp2, idist2=idist2)
-        rc = _lib.load().mufft_hip_execute_plan_1d_mul_batched(
+        idist2 = 0 applies one inp2 block to every transform; head: only the first
+        half of each output is written (up to 65536 complex points)."""
+        self._validate(out, inp, howmany, idist, odist, adjoint=adjoint, inp2=inp2, idist2=idist2, head=head)
+        L = _lib.load()
+        fn = L.mufft_hip_execute_plan_1d_mul_head_batched if head else L.mufft_hip_execute_plan_1d_mul_batched
+        rc = fn(
             self._h, ptr(out), ptr(inp), ptr(inp2), howmany, idist, idist2, odist,
             ctypes.c_float(norm), int(conj2), int(adjoint), stream_handle(stream))
         _check(rc, "mufft_hip_execute_plan_1d_mul_batched")
@@ -354,6 +359,8 @@ class ConvBatch:
         self._h = h
 
     def execute(self, stream=None, graph: bool = True):
+        """One launch of the batch's kernel; ``graph`` selects the entry point of
+        that name, which does the same."""
         L = _lib.load()
         fn = L.mufft_hip_execute_conv_batch if graph else L.mufft_hip_execute_conv_batch_direct
         _check(fn(self._h, stream_handle(stream)), "mufft_hip_execute_conv_batch")
