@@ -40,6 +40,8 @@ class FFTConv:
             self.p_second = A.Plan1D("r2c", N, flags=zp)
             self.p_out = A.Plan1D("c2r", N)
             self.nbins = N // 2 + 1
+        # Fused kernels store the kept half of the input gradient alone.
+        self.head_out = (N if stereo else N // 2) <= 65536
 
     def __call__(self, x: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
         return _ConvFn.apply(x, h, self)
@@ -75,10 +77,16 @@ class _ConvFn(torch.autograd.Function):
         op.p_out.execute_adjoint_batched(G, dy, B, stream=s)
         dx = dh = None
         if ctx.needs_input_grad[0]:
-            full = torch.empty((B, N), dtype=torch.complex64 if op.stereo else torch.float32, device=dev)
-            op.p_first.execute_mul_batched(full, G, H, B, idist2=0, norm=1.0 / N, conj2=True,
-                                           adjoint=True, stream=s)
-            dx = full[:, : N // 2].contiguous()
+            dtype = torch.complex64 if op.stereo else torch.float32
+            if op.head_out:
+                dx = torch.empty((B, N // 2), dtype=dtype, device=dev)
+                op.p_first.execute_mul_batched(dx, G, H, B, idist2=0, norm=1.0 / N, conj2=True,
+                                               adjoint=True, stream=s, head=True)
+            else:
+                full = torch.empty((B, N), dtype=dtype, device=dev)
+                op.p_first.execute_mul_batched(full, G, H, B, idist2=0, norm=1.0 / N, conj2=True,
+                                               adjoint=True, stream=s)
+                dx = full[:, : N // 2].contiguous()
         if ctx.needs_input_grad[1]:
             dH = torch.empty((1, op.nbins), dtype=torch.complex64, device=dev)
             A.mul_reduce(dH, G, X, op.nbins, B, norm=1.0 / N, conj_b=True, stream=s)

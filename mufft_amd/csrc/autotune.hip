@@ -411,7 +411,8 @@ int mufft_hip_get_large_split(unsigned N, int kind) {
         set_err("no split for this size");
         return -1;
     }
-    return chosen_fs_code(l);
+    const int tk = tk_from_api(kind);
+    return chosen_fs_code(l, tk == TK_R2C ? KIND_R2C : (tk == TK_C2R ? KIND_C2R : KIND_C2C));
 }
 
 int mufft_hip_set_large_split(unsigned N, int kind, int code) {

@@ -29,10 +29,12 @@ enum RowFlag : unsigned {
     // The next kernel reads the output: store it cacheable (default: streaming
     // stores, for outputs that leave the device's caches anyway).
     RF_KEEP_OUT = 1u << 6,
+    // c2c / c2r store only the first half of their output.
+    RF_HEAD_OUT = 1u << 7,
 };
 // Every flag: a launch with none of them runs the kernels' plain
 // instantiation, where the flags are compile-time zero.
-constexpr unsigned RF_ALL = (1u << 7) - 1u;
+constexpr unsigned RF_ALL = (1u << 8) - 1u;
 // Template argument of the fused transforms: flags read at run time (any
 // other value fixes them at compile time).
 constexpr unsigned RF_DYNAMIC = ~0u;
@@ -135,6 +137,22 @@ MUFFT_HD constexpr int rv_default_base(int N, int kind) {
          : rv_make_split(1, rv_make(32, 1, 1));
 }
 MUFFT_HD constexpr int rv_default(int N, int kind = 0) { return rv_default_base(N, kind); }
+// Flag sets that the default variants also run with their flags fixed, beside
+// none: the halves of the block convolution and of its gradients (zero-padded
+// inputs; multiply; conjugated multiply of an adjoint, first half kept).  With
+// the flags read at run time a uniform branch per point splits the loads and
+// stores: c2c 65536 x 64 with the multiply 42.5 -> 35.8 us, zero-padded 31.3 ->
+// 29.4.
+MUFFT_HD constexpr unsigned rf_fixed(int kind, int dir, int i) {
+    return kind == KIND_R2C ? (i == 0 ? RF_ZERO_PAD : RF_ADJ_C2R)
+         : kind == KIND_C2R ? (i == 0 ? RF_MUL : RF_MUL | RF_CONJ2 | RF_ADJ_R2C | RF_HEAD_OUT)
+         : dir < 0 ? (unsigned)RF_ZERO_PAD
+         : (i == 0 ? RF_MUL : RF_MUL | RF_CONJ2 | RF_HEAD_OUT);
+}
+// Whether a variant is the default of its size and kind, and so carries them.
+MUFFT_HD constexpr bool rf_fixed_variant(int N, int dir, int kind, int var) {
+    return var == rv_default(N, kind == KIND_R2C ? 2 : (kind == KIND_C2R ? 3 : 0));
+}
 
 // Radix sequence of NP passes: NP - 1 passes of radix R and one of the
 // remainder N / R^(NP-1), placed first (REM_FIRST) or last.  The twiddle
@@ -191,6 +209,9 @@ MUFFT_HD constexpr int col_TX_alt(int L, int i = 0) {
                   : (i == 1 && L == 4096 ? 4 : 0);   // at 512-4096 points one is half the default
 }
 constexpr int COL_TX_ALTS = 2;
+// The width the library reports for a length where none is set (512, 2048 and
+// 4096 points: the narrower of the two that launches choose between).
+MUFFT_HD constexpr int col_TX_nominal(int L) { return L == 512 || L == 2048 || L == 4096 ? col_TX(L) / 2 : col_TX(L); }
 // The width a plain launch over `images` of `ncols` columns takes: where full
 // tiles are at most 128, half the CUs, the half-width ones fill more of the
 // GPU (2D c2c, us: 1024 x 512 x 1 12.8 -> 11.9, 1024^2 x 1 17.0 -> 15.7, 512 x
@@ -301,7 +322,7 @@ constexpr int COL_MAX_LOG2 = 13;   // fused column kernel covers L <= 8192
 MUFFT_HD constexpr int fs3_split(int logn) {
     return logn == 23 ? (9 << 8) | (8 << 4) | 6
          : logn == 24 ? (10 << 8) | (8 << 4) | 6
-         : logn == 25 ? (9 << 8) | (8 << 4) | 8
+         : logn == 25 ? (9 << 8) | (10 << 4) | 6
          : logn == 26 ? (10 << 8) | (10 << 4) | 6
          : 0;
 }
@@ -323,11 +344,26 @@ MUFFT_HD constexpr bool fs_code_valid(int logn, int code) {
              fs_code_b(code) <= 10 && fs_code_n1(code) + fs_code_a(code) + fs_code_b(code) == logn));
 }
 MUFFT_HD constexpr int fs_log_n1(int logn) {
-    return logn == 17 ? 9 : logn == 18 ? 8 : logn == 21 ? 11 : logn == 22 ? 12 : logn == 23 ? 11
+    return logn == 17 || logn == 18 ? 9 : logn == 21 ? 11 : logn == 22 ? 12 : logn == 23 ? 11
          : logn == 25 ? 13 : logn / 2;
 }
-MUFFT_HD constexpr int fs_code_default(int logn) {
-    return fs3_split(logn) ? fs3_split(logn) : (fs_log_n1(logn) << 8);
+// Per transform kind (KIND_*), where the real transforms' fused launches
+// (real_cols.hip) have another best split: r2c resolves in the last launch and
+// prefers it short, c2r in the first, of 256 to 1024 points.  From a sweep of
+// every split at 256 MiB of reals, us, the c2c split against these: r2c 2^18
+// complex 305 / 262, 2^19 305 / 288, 2^20 327 / 313, 2^22 337 / 319, 2^24 346 /
+// 338, 2^25 372 / 343; c2r 2^17 229 / 211, 2^18 225 / 213, 2^21 390 / 308, 2^22
+// 424 / 332, 2^24 393 / 367, 2^25 370 / 360.
+MUFFT_HD constexpr int fs_code_default(int logn, int kind = KIND_C2C) {
+    return kind == KIND_R2C && (logn == 18 || logn == 20) ? 12 << 8
+         : kind == KIND_R2C && logn == 19 ? 11 << 8
+         : kind == KIND_R2C && logn == 22 ? (10 << 8) | (6 << 4) | 6
+         : kind == KIND_R2C && logn == 24 ? (8 << 8) | (10 << 4) | 6
+         : kind == KIND_R2C && logn == 25 ? (10 << 8) | (8 << 4) | 7
+         : kind == KIND_C2R && (logn == 17 || logn == 18) ? 8 << 8
+         : kind == KIND_C2R && (logn == 21 || logn == 22) ? 10 << 8
+         : kind == KIND_C2R && logn == 24 ? (8 << 8) | (8 << 4) | 8
+         : fs3_split(logn) ? fs3_split(logn) : (fs_log_n1(logn) << 8);
 }
 constexpr int ROW_MAX_LOG2 = 16;   // fused row kernels (one or two workgroups per transform) cover N <= 65536
 constexpr int ROW_WG_MAX_LOG2 = 15;  // one workgroup per transform up to 32768 points

@@ -137,9 +137,9 @@ void set_chosen_variant(int logn, int tk, int variant);
 // Whether a size has a tuned or explicitly set choice.
 bool variant_is_set(int logn, int tk);
 // Process-wide split of transforms of 2^logn points beyond the fused sizes
-// (a fs_code; 0 = the static fs_code_default) and tile width of the column
-// kernel of 2^logL points (0 = col_TX): the autotuner's or an explicit choice.
-int chosen_fs_code(int logn);
+// (a fs_code for every kind; 0 = the static fs_code_default of the kind) and tile width of the column
+// kernel of 2^logL points (0: by launch, col_TX_for; reported as col_TX_nominal): the autotuner's or an explicit choice.
+int chosen_fs_code(int logn, int kind);
 void set_fs_code(int logn, int code);
 int chosen_col_tx(int logL);
 int set_col_tx_or_0(int logL);   // 0: not set, the static choice

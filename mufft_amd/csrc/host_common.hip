@@ -192,7 +192,8 @@ bool variant_is_set(int logn, int tk) {
 namespace {
 constexpr bool default_splits_valid() {
     for (int l = ROW_MAX_LOG2 + 1; l <= 2 * COL_MAX_LOG2; ++l)
-        if (!fs_code_valid(l, fs_code_default(l))) return false;
+        for (int kind : {KIND_C2C, KIND_R2C, KIND_C2R})
+            if (!fs_code_valid(l, fs_code_default(l, kind))) return false;
     return true;
 }
 static_assert(default_splits_valid(), "every static split of the four-step sizes is runnable");
@@ -200,10 +201,10 @@ int g_fs_code[2 * COL_MAX_LOG2 + 1] = {};
 int g_col_tx[COL_MAX_LOG2 + 1] = {};
 }  // namespace
 
-int chosen_fs_code(int logn) {
+int chosen_fs_code(int logn, int kind) {
     std::lock_guard<std::mutex> g(g_var_lock);
     const int c = (logn >= 0 && logn <= 2 * COL_MAX_LOG2) ? g_fs_code[logn] : 0;
-    return c ? c : fs_code_default(logn);
+    return c ? c : fs_code_default(logn, kind);
 }
 
 void set_fs_code(int logn, int code) {
@@ -218,7 +219,7 @@ int set_col_tx_or_0(int logL) {
 
 int chosen_col_tx(int logL) {
     const int t = set_col_tx_or_0(logL);
-    return t ? t : col_TX(1 << logL);
+    return t ? t : col_TX_nominal(1 << logL);
 }
 
 void set_col_tx(int logL, int tx) {
@@ -242,7 +243,7 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         if (build_stockham_table(n, dir, fused_sequence(n, col_E(n), false), &tw_col, s)) return -1;
     }
     if (rows && four_step()) {
-        fs_code = fs ? fs : chosen_fs_code(logn);
+        fs_code = fs ? fs : chosen_fs_code(logn, kind);
         if (!fs_code_valid(logn, fs_code)) {
             set_err("split %#x is not valid for 2^%d points", fs_code, logn);
             return -1;

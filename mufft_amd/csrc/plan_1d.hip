@@ -155,8 +155,11 @@ static int ensure_adjoint(mufft_plan_1d *p) {
 static int exec_adjoint(mufft_plan_1d *p, void *out, const void *in, const void *in2,
                         unsigned howmany, long long idist, long long idist2, long long odist,
                         unsigned extra, float norm, hipStream_t st) {
-    return with_scratch(p->scratch, st, [&]() -> int {
+    {
+        std::lock_guard<std::mutex> g(p->scratch.m);
         if (ensure_adjoint(p)) return -1;
+    }
+    auto run = [&]() -> int {
         int kind, dir;
         unsigned fl;
         adjoint_shape(p, &kind, &dir, &fl);
@@ -185,7 +188,11 @@ static int exec_adjoint(mufft_plan_1d *p, void *out, const void *in, const void 
         return run_rows(p->adj, kind, rtw, src, sd, static_cast<const float2 *>(in2), idist2,
                         static_cast<float2 *>(out), odist, (int)howmany, fl | extra, norm, p->s0,
                         p->s1, st);
-    });
+    };
+    // As in exec_1d: the fused kernels touch no plan-owned buffer but the
+    // read-only tables, so they need no ordering with other streams' calls.
+    if (!rows_use_scratch(p->adj) && !(p->kind == KIND_R2C && p->full)) return run();
+    return with_scratch(p->scratch, st, run);
 }
 
 void exec_1d_dropin(mufft_plan_1d *p, void *out, const void *in, const void *in2, size_t in2_bytes,
@@ -354,10 +361,9 @@ int mufft_hip_execute_adjoint_1d_batched(mufft_plan_1d *p, void *output, const v
                         static_cast<hipStream_t>(stream));
 }
 
-int mufft_hip_execute_plan_1d_mul_batched(mufft_plan_1d *p, void *output, const void *input,
-                                          const void *input2, unsigned howmany, size_t idist,
-                                          size_t idist2, size_t odist, float norm, int conj2,
-                                          int adjoint, void *stream) {
+static int exec_mul(mufft_plan_1d *p, void *output, const void *input, const void *input2, unsigned howmany,
+                    size_t idist, size_t idist2, size_t odist, float norm, int conj2, int adjoint, bool head,
+                    void *stream) {
     if (!p || !output || !input || !input2) {
         set_err("null argument");
         return -1;
@@ -369,14 +375,33 @@ int mufft_hip_execute_plan_1d_mul_batched(mufft_plan_1d *p, void *output, const 
         set_err("no fused multiply for transforms with real input");
         return -1;
     }
+    if (head && !p->eng.row_fused()) {
+        set_err("the first half alone is stored only up to %d complex points", 1 << ROW_MAX_LOG2);
+        return -1;
+    }
     long long id, od;
     if (api_dists(p, adjoint != 0, idist, odist, &id, &od) || kernel_ptrs(&output, &input, &input2))
         return -1;
-    const unsigned extra = RF_MUL | (conj2 ? RF_CONJ2 : 0u);
+    if (head && odist == 0) od /= 2;   // packed halves
+    const unsigned extra = RF_MUL | (conj2 ? RF_CONJ2 : 0u) | (head ? RF_HEAD_OUT : 0u);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (adjoint)
         return exec_adjoint(p, output, input, input2, howmany, id, (long long)idist2, od, extra, norm, st);
     return exec_1d(p, output, input, input2, howmany, id, (long long)idist2, od, extra, norm, st);
+}
+
+int mufft_hip_execute_plan_1d_mul_batched(mufft_plan_1d *p, void *output, const void *input,
+                                          const void *input2, unsigned howmany, size_t idist,
+                                          size_t idist2, size_t odist, float norm, int conj2,
+                                          int adjoint, void *stream) {
+    return exec_mul(p, output, input, input2, howmany, idist, idist2, odist, norm, conj2, adjoint, false, stream);
+}
+
+int mufft_hip_execute_plan_1d_mul_head_batched(mufft_plan_1d *p, void *output, const void *input,
+                                               const void *input2, unsigned howmany, size_t idist,
+                                               size_t idist2, size_t odist, float norm, int conj2,
+                                               int adjoint, void *stream) {
+    return exec_mul(p, output, input, input2, howmany, idist, idist2, odist, norm, conj2, adjoint, true, stream);
 }
 
 int mufft_hip_plan_1d_launches(const mufft_plan_1d *p) {

@@ -54,11 +54,12 @@ __device__ __forceinline__ void row_transform(const float2 *X, const float2 *Y, 
     const bool cj = (flags & RF_CONJ2) != 0;
     const bool full = (flags & RF_FULL) != 0;
     const bool adj = (flags & (RF_ADJ_R2C | RF_ADJ_C2R)) != 0;
+    const bool head = (flags & RF_HEAD_OUT) != 0;
     // Element vp + sp of an operand: vp per lane, sp a compile-time slot offset.
     __amdgpu_buffer_rsrc_t rin, rin2, rout, rrtw;  // set and used only when BUF
     if constexpr (BUF) {
         const unsigned nin = KIND == KIND_C2R ? N + 1 : ((zp && !mul) ? N / 2 : N);
-        const unsigned nout = KIND == KIND_R2C ? (full ? 2 * N : N + 1) : N;
+        const unsigned nout = KIND == KIND_R2C ? (full ? 2 * N : N + 1) : (head ? N / 2 : N);
         rin = make_rsrc(X, active ? nin * 8u : 0u);
         rin2 = make_rsrc(Y, (active && mul) ? (KIND == KIND_C2R ? N + 1 : N) * 8u : 0u);
         rout = make_rsrc(Xo, active ? nout * 8u : 0u);
@@ -264,7 +265,7 @@ __device__ __forceinline__ void row_transform(const float2 *X, const float2 *Y, 
         if (BUF || active) {
             static_for<0, E>([&](auto C) {
                 constexpr int c = decltype(C)::value;
-                st_out(lt, T * c, v[c]);
+                if (!(head && c >= E / 2)) st_out(lt, T * c, v[c]);
             });
         }
     }
@@ -284,26 +285,25 @@ __global__ void __launch_bounds__(rv_WG(N, VAR), rv_waves_per_simd(N, VAR)) fft_
     const long long g = (long long)blockIdx.x * B + sub;
     // r2c stores cacheable anyway: RF_KEEP_OUT changes nothing there.
     constexpr unsigned MOOT = KIND == KIND_R2C ? (unsigned)RF_KEEP_OUT : 0u;
-    if ((a.flags & RF_ALL & ~MOOT) == 0) {
-        row_transform<N, DIR, KIND, VAR, MOOT>(a.in + g * a.idist, a.in2 + g * a.idist2, a.out + g * a.odist,
-                                               g < a.batch, lt, a.tw, a.rtw, 0u, a.norm, smem + sub * LDSN,
-                                               reinterpret_cast<float *>(smem) + sub * LDSN);
-        return;
-    }
+    const unsigned flags = a.flags & RF_ALL;
+    auto run = [&](auto FIXED) {
+        row_transform<N, DIR, KIND, VAR, decltype(FIXED)::value>(
+            a.in + g * a.idist, a.in2 + g * a.idist2, a.out + g * a.odist, g < a.batch, lt, a.tw, a.rtw, flags,
+            a.norm, smem + sub * LDSN, reinterpret_cast<float *>(smem) + sub * LDSN);
+    };
+    if ((flags & ~MOOT) == 0) return run(std::integral_constant<unsigned, MOOT>{});
     if constexpr (KIND == KIND_C2C) {
         // The 2D row pass (its output is read by the column pass): 2D c2c
         // 1024^2 x 16 -3% to -6% with the flag fixed.
-        if ((a.flags & RF_ALL) == RF_KEEP_OUT) {
-            row_transform<N, DIR, KIND, VAR, RF_KEEP_OUT>(a.in + g * a.idist, a.in2 + g * a.idist2,
-                                                          a.out + g * a.odist, g < a.batch, lt, a.tw, a.rtw,
-                                                          a.flags, a.norm, smem + sub * LDSN,
-                                                          reinterpret_cast<float *>(smem) + sub * LDSN);
-            return;
-        }
+        if (flags == RF_KEEP_OUT) return run(std::integral_constant<unsigned, RF_KEEP_OUT>{});
     }
-    row_transform<N, DIR, KIND, VAR>(a.in + g * a.idist, a.in2 + g * a.idist2, a.out + g * a.odist, g < a.batch,
-                                     lt, a.tw, a.rtw, a.flags, a.norm, smem + sub * LDSN,
-                                     reinterpret_cast<float *>(smem) + sub * LDSN);
+    if constexpr (rf_fixed_variant(N, DIR, KIND, VAR)) {
+        constexpr unsigned f0 = rf_fixed(KIND, DIR, 0), f1 = rf_fixed(KIND, DIR, 1);
+        if ((flags & ~MOOT) == f0) return run(std::integral_constant<unsigned, f0 | MOOT>{});
+        if constexpr (f1 != f0)
+            if ((flags & ~MOOT) == f1) return run(std::integral_constant<unsigned, f1 | MOOT>{});
+    }
+    run(std::integral_constant<unsigned, RF_DYNAMIC>{});
 }
 
 // Entries [I, END) of the table of the instantiated variants of one

@@ -52,9 +52,10 @@ __device__ __forceinline__ void split_transform(const float2 *X, const float2 *Y
     const bool cj = (flags & RF_CONJ2) != 0;
     const bool full = (flags & RF_FULL) != 0;
     const bool adj = (flags & (RF_ADJ_R2C | RF_ADJ_C2R)) != 0;
+    const bool head = (flags & RF_HEAD_OUT) != 0;
 
     const unsigned nin = KIND == KIND_C2R ? NT + 1 : ((zp && !mul) ? NT / 2 : NT);
-    const unsigned nout = KIND == KIND_R2C ? (full ? 2 * NT : NT + 1) : NT;
+    const unsigned nout = KIND == KIND_R2C ? (full ? 2 * NT : NT + 1) : (head ? NT / 2 : NT);
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(X, nin * 8u);
     const __amdgpu_buffer_rsrc_t rin2 = make_rsrc(Y, mul ? (KIND == KIND_C2R ? NT + 1 : NT) * 8u : 0u);
     const __amdgpu_buffer_rsrc_t rout = make_rsrc(Xo, nout * 8u);
@@ -212,7 +213,7 @@ __device__ __forceinline__ void split_transform(const float2 *X, const float2 *Y
     if constexpr (KIND != KIND_R2C) {
         static_for<0, E>([&](auto C) {
             constexpr int c = decltype(C)::value;
-            bstore(rout, (unsigned)(N1 * lt) * 8u, (unsigned)(N1 * T * c + k1) * 8u, v[c]);
+            if (!(head && c >= E / 2)) bstore(rout, (unsigned)(N1 * lt) * 8u, (unsigned)(N1 * T * c + k1) * 8u, v[c]);
         });
     } else {
         // Bin k = 2*k2 + k1 needs Z[k] and Z[NT - k], which is v at
@@ -266,14 +267,20 @@ __global__ void __launch_bounds__(rv_T(N2, VAR), rv_waves_per_simd(N2, VAR)) fft
     const long long t = g / N1;
     const int k1 = (int)(g % N1);
     // The split's stores are cacheable anyway: RF_KEEP_OUT changes nothing.
-    if ((a.flags & RF_ALL & ~(unsigned)RF_KEEP_OUT) == 0)
-        split_transform<N2, N1, DIR, KIND, VAR, 0u>(a.in + t * a.idist, a.in2 + t * a.idist2, a.out + t * a.odist,
-                                                      k1, threadIdx.x, a.tw, a.stw, a.rtw, 0u, a.norm, smem,
-                                                      reinterpret_cast<float *>(smem));
-    else
-        split_transform<N2, N1, DIR, KIND, VAR>(a.in + t * a.idist, a.in2 + t * a.idist2, a.out + t * a.odist,
-                                                k1, threadIdx.x, a.tw, a.stw, a.rtw, a.flags, a.norm, smem,
-                                                reinterpret_cast<float *>(smem));
+    const unsigned flags = a.flags & RF_ALL & ~(unsigned)RF_KEEP_OUT;
+    auto run = [&](auto FIXED) {
+        split_transform<N2, N1, DIR, KIND, VAR, decltype(FIXED)::value>(
+            a.in + t * a.idist, a.in2 + t * a.idist2, a.out + t * a.odist, k1, threadIdx.x, a.tw, a.stw, a.rtw, flags,
+            a.norm, smem, reinterpret_cast<float *>(smem));
+    };
+    if (flags == 0) return run(std::integral_constant<unsigned, 0u>{});
+    if constexpr (rf_fixed_variant(N1 * N2, DIR, KIND, rv_make_split(ilog2(N1), VAR))) {
+        constexpr unsigned f0 = rf_fixed(KIND, DIR, 0), f1 = rf_fixed(KIND, DIR, 1);
+        if (flags == f0) return run(std::integral_constant<unsigned, f0>{});
+        if constexpr (f1 != f0)
+            if (flags == f1) return run(std::integral_constant<unsigned, f1>{});
+    }
+    run(std::integral_constant<unsigned, RF_DYNAMIC>{});
 }
 
 }  // namespace mufft
