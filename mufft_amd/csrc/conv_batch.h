@@ -11,8 +11,17 @@ constexpr int CB_WG = 1024;           // threads per workgroup of the persistent
 constexpr int CB_LDS_BYTES = 139264;  // 1024 threads x 17 padded points x 8 bytes
 constexpr int CB_MIN_LOG2 = 2;        // smallest fused transform inside the kernel (4 points)
 constexpr int CB_SPLIT_LOG2 = 15;     // 32768 points: two workgroups per transform
+// Jobs that run whole in one task, by the points of their transforms: mono ones
+// whose threads lie in one wave (no workgroup barrier; 57 jobs of 1024 reals
+// 43 -> 31 us), stereo ones up to what a workgroup holds (128 jobs of 16384
+// points 70 -> 65 us, 256 87 -> 75).  Larger mono jobs run as fast or faster in
+// parts: whole, the three resolves' exchanges and spills cost what the saved
+// spectra gain (57 jobs of 32768 reals 57 -> 76 us).
+MUFFT_HD constexpr bool cb_whole_job(int logn, bool stereo) { return logn <= (stereo ? 14 : 10); }
 
-enum CBTaskType : int { CB_FWD_FIRST = 0, CB_FWD_SECOND = 1, CB_INV = 2 };
+// CB_JOB: both forward transforms, the product and the inverse transform of
+// its jobs; the other three are the parts of a larger job.
+enum CBTaskType : int { CB_FWD_FIRST = 0, CB_FWD_SECOND = 1, CB_INV = 2, CB_JOB = 3 };
 
 // One convolution job: device pointers of its inputs, spectra and output.
 struct CBJob {
@@ -28,13 +37,14 @@ constexpr int CB_XCDS = 8;
 // A group of up to CB_WG / T jobs sharing one transform shape.
 struct CBTask {
     int type;              // CBTaskType
-    int kind;              // KIND_C2C / KIND_R2C / KIND_C2R
+    int kind;              // KIND_C2C / KIND_R2C / KIND_C2R; CB_JOB: KIND_C2C stereo, KIND_R2C mono
     int dir;               // -1 forward, +1 inverse
     int logn;              // log2 of the fused (complex) transform length
     int job0, njobs;       // jobs [job0, job0 + njobs) of the job table
-    unsigned flags;        // RowFlag bits
+    unsigned flags;        // RowFlag bits; CB_JOB: bit 0 / 1: the first / second input is zero padded
     float norm;            // 1/N for the inverse multiply
-    const float2 *tw;      // Stockham twiddles of the transform
+    const float2 *tw;      // Stockham twiddles of the transform (CB_JOB: the forward ones)
+    const float2 *tw_inv;  // CB_JOB: the inverse ones
     const float2 *rtw;     // real-transform resolve twiddles (r2c / c2r)
     // Transforms of 2^CB_SPLIT_LOG2 points run as two workgroup tasks
     // (k1 = 0, 1) of the split transform (split_impl.h); stw is its twiddle table.
@@ -44,7 +54,8 @@ struct CBTask {
     int nprod;             // inverse tasks: forward tasks the group needs first
 };
 
-// One persistent launch runs the whole batch.  Each job group (the jobs of
+// One persistent launch runs the whole batch.  Jobs of cb_whole_job sizes run
+// whole, a task for as many as a workgroup holds; the others in parts.  Each job group (the jobs of
 // one task shape) is assigned to one XCD, and that XCD's workgroups (read
 // from the hardware XCC_ID register) pull its tasks from the XCD's own
 // queue: first the forward tasks, then the inverse tasks.  A forward task

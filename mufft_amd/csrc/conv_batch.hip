@@ -110,20 +110,176 @@ __device__ __noinline__ void cb_run(const CBTask &t, const CBJob *__restrict__ j
     cb_run_fl<KIND, DIR, LOGN, RF_DYNAMIC>(t, jobs, tid, smem);
 }
 
-template <int KIND, int DIR, int LO, int HI>
-__device__ __forceinline__ void cb_dispatch_sizes(const CBTask &t, const CBJob *jobs, int tid,
-                                                  float2 *smem) {
-    static_for<LO, HI + 1>([&](auto L) {
-        if (t.logn == decltype(L)::value) cb_run<KIND, DIR, decltype(L)::value>(t, jobs, tid, smem);
+// A pointer to global memory (its accesses are global, not flat, ones).
+template <typename P>
+struct CBGlobal {
+    typedef __attribute__((address_space(1))) P *Ptr;
+    Ptr p;
+    __device__ __forceinline__ explicit CBGlobal(P *q) : p((Ptr)(uintptr_t)q) {}
+    __device__ __forceinline__ std::remove_const_t<P> load(int i) const {
+        if constexpr (sizeof(P) == 8) {
+            const float x = ((__attribute__((address_space(1))) const float *)p)[2 * i];
+            const float y = ((__attribute__((address_space(1))) const float *)p)[2 * i + 1];
+            return make_float2(x, y);
+        } else {
+            return p[i];
+        }
+    }
+    __device__ __forceinline__ void store(int i, float2 v) const {
+        ((__attribute__((address_space(1))) float *)p)[2 * i] = v.x;
+        ((__attribute__((address_space(1))) float *)p)[2 * i + 1] = v.y;
+    }
+};
+
+// Whole jobs (CB_JOB, cb_whole_job): both inputs' forward passes, the product
+// and the inverse passes with the points in registers.  In three tasks a job
+// writes and reads its spectra and waits for its own group; whole, it takes one
+// load and one store.  Bound by the latency of its chain of passes.  Stereo: the filter runs as a complex transform of zero imaginary part,
+// so the product needs no other point.  Mono: the resolves (kernel.c:36-82)
+// pair points k and N-k through LDS.
+template <int LOGN, bool STEREO>
+__device__ __noinline__ void cb_run_job(const CBTask &t, const CBJob *__restrict__ jobs, int tid, float2 *smem) {
+    constexpr int N = 1 << LOGN;
+    constexpr int VAR = cb_variant(N);
+    constexpr int E = rv_E(N, VAR);
+    constexpr int LOGE = ilog2(E);
+    constexpr int T = rv_T(N, VAR);
+    constexpr int TWM = rv_twm(VAR);
+    constexpr bool WAVE = T <= 64;
+    static_assert(cb_lds_bytes(N) <= CB_LDS_BYTES, "LDS budget of the persistent kernel");
+    constexpr bool BUF = T >= 64;   // a wave lies in one job: descriptors, one offset per lane
+    const int lt = tid & (T - 1);
+    const int sub = BUF ? __builtin_amdgcn_readfirstlane(tid / T) : tid / T;
+    const bool active = sub < t.njobs;
+    if (WAVE && !active) return;   // no barrier of the workgroup inside
+    const CBJob &j = jobs[t.job0 + (active ? sub : 0)];
+    float2 *L = smem + sub * rv_lds_per(N, VAR);
+    auto slot = [](int o) { return pad_slot<LOGE>(o); };
+    const bool zp1 = (t.flags & 1u) != 0, zp2 = (t.flags & 2u) != 0;
+
+    // The pointers come from memory: cast to the global address space, or the
+    // accesses would be flat ones, which wait for the LDS as well.
+    __amdgpu_buffer_rsrc_t rin1, rin2, rout;
+    const CBGlobal<const float2> g1(j.first), g2(j.second);
+    const CBGlobal<float2> go(j.out);
+    if constexpr (BUF) {
+        // Zero padding and idle slots by the descriptors' bounds.
+        rin1 = make_rsrc(j.first, active ? (zp1 ? N / 2 : N) * 8u : 0u);
+        rin2 = make_rsrc(j.second, active ? (zp2 ? N / 2 : N) * (STEREO ? 4u : 8u) : 0u);
+        rout = make_rsrc(j.out, active ? N * 8u : 0u);
+    }
+    float2 u[E], v[E];
+    static_for<0, E>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        if constexpr (BUF) u[c] = bload_nt(rin1, (unsigned)lt * 8u, T * c * 8u);
+        else u[c] = !(zp1 && c >= E / 2) ? g1.load(lt + T * c) : make_float2(0.f, 0.f);
+    });
+    static_for<0, E>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        if constexpr (STEREO && BUF) {
+            v[c] = make_float2(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rin2, lt * 4, T * c * 4, 2)), 0.f);
+        } else if constexpr (STEREO) {
+            const CBGlobal<const float> f2(reinterpret_cast<const float *>(j.second));
+            v[c] = make_float2(!(zp2 && c >= E / 2) ? f2.load(lt + T * c) : 0.f, 0.f);
+        } else if constexpr (BUF) {
+            v[c] = bload_nt(rin2, (unsigned)lt * 8u, T * c * 8u);
+        } else {
+            v[c] = !(zp2 && c >= E / 2) ? g2.load(lt + T * c) : make_float2(0.f, 0.f);
+        }
+    });
+    auto passes = [&](auto DIR, float2(&z)[E]) {
+        constexpr int dir = decltype(DIR)::value;
+        const float2 *tw = dir < 0 ? t.tw : t.tw_inv;
+        if constexpr (BUF) {
+            constexpr unsigned ntw = (unsigned)(N - seq_first(N, E, np_for(N, E), true));
+            stockham_passes<N, E, dir, XM_PAD, TWM, E, WAVE, true>(z, lt, TwBuffer{make_rsrc(tw, ntw * 8u)}, L, nullptr, slot);
+        } else {
+            const CBGlobal<const float2> g(tw);
+            stockham_passes<N, E, dir, XM_PAD, TWM, E, WAVE, true>(
+                z, lt, [&](int idx, int k) { return g.load(idx + k); }, L, nullptr, slot);
+        }
+    };
+    constexpr std::integral_constant<int, -1> FWD;
+    constexpr std::integral_constant<int, 1> INV;
+    passes(FWD, u);
+    if constexpr (STEREO) {
+        passes(FWD, v);
+        static_for<0, E>([&](auto C) {
+            constexpr int c = decltype(C)::value;
+            u[c] = cscale(cmul(u[c], v[c]), t.norm);
+        });
+    } else {
+        // Point N - k of every point k = lt + T*c, through LDS (point 0 its own).
+        auto partners = [&](const float2(&z)[E], auto use) {
+            static_for<0, E>([&](auto C) { L[slot(lt + T * decltype(C)::value)] = z[decltype(C)::value]; });
+            exchange_sync<WAVE>();
+            static_for<0, E>([&](auto C) {
+                constexpr int c = decltype(C)::value;
+                use(C, L[slot((N - lt - T * c) & (N - 1))]);
+            });
+            exchange_sync<WAVE>();
+        };
+        // W[k] = -i exp(-i pi k / N): one entry per thread and constant rotations.
+        const float2 w0 = CBGlobal<const float2>(t.rtw).load(lt);
+        // r2c resolve; thread 0's point 0 becomes (X[0], X[N]), both real.
+        auto resolve = [&](float2(&z)[E]) {
+            partners(z, [&](auto C, float2 p) {
+                constexpr int c = decltype(C)::value;
+                const float2 za = z[c], zb = cconj(p);
+                const float2 x = cscale(cadd(cadd(za, zb), cmul(twc<c, 2 * E, -1>(w0), csub(za, zb))), 0.5f);
+                z[c] = c == 0 && lt == 0 ? make_float2(za.x + za.y, za.x - za.y) : x;
+            });
+        };
+        resolve(u);
+        passes(FWD, v);
+        resolve(v);
+        static_for<0, E>([&](auto C) {
+            constexpr int c = decltype(C)::value;
+            const float2 y = c == 0 && lt == 0 ? make_float2(u[c].x * v[c].x, u[c].y * v[c].y) : cmul(u[c], v[c]);
+            u[c] = cscale(y, t.norm);
+        });
+        // c2r resolve, W'[k] = conj(W[k]).
+        partners(u, [&](auto C, float2 p) {
+            constexpr int c = decltype(C)::value;
+            const float2 ya = u[c], yb = cconj(p);
+            const float2 z = cadd(cadd(ya, yb), cmul(csub(ya, yb), cconj(twc<c, 2 * E, -1>(w0))));
+            u[c] = c == 0 && lt == 0 ? make_float2(ya.x + ya.y, ya.x - ya.y) : z;
+        });
+    }
+    passes(INV, u);
+    static_for<0, E>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        if constexpr (BUF) bstore_nt(rout, (unsigned)lt * 8u, T * c * 8u, u[c]);
+        else go.store(lt + T * c, u[c]);
     });
 }
 
 template <int KIND_, int DIR_>
 __device__ __forceinline__ void cb_dispatch_kind(const CBTask &t, const CBJob *jobs, int tid, float2 *smem) {
-    cb_dispatch_sizes<KIND_, DIR_, CB_MIN_LOG2, 15>(t, jobs, tid, smem);
+    static_for<CB_MIN_LOG2, CB_SPLIT_LOG2 + 1>([&](auto L) {
+        constexpr int l = decltype(L)::value;
+        // Parts of the jobs that do not run whole: mono ones of l points, or
+        // the stereo ones (whose filter's spectrum has half the points).
+        constexpr bool used = KIND_ == KIND_C2C ? !cb_whole_job(l, true)
+                                                : !cb_whole_job(l, false) || (KIND_ == KIND_R2C && !cb_whole_job(l + 1, true));
+        if constexpr (used)
+            if (t.logn == l) cb_run<KIND_, DIR_, l>(t, jobs, tid, smem);
+    });
 }
 
 __device__ __forceinline__ void cb_run_task(const CBTask &t, const CBJob *jobs, int tid, float2 *smem) {
+    if (t.type == CB_JOB) {
+        static_for<CB_MIN_LOG2, CB_SPLIT_LOG2>([&](auto L) {
+            constexpr int l = decltype(L)::value;
+            if (t.logn != l) return;
+            if (t.kind == KIND_C2C) {
+                if constexpr (cb_whole_job(l, true)) cb_run_job<l, true>(t, jobs, tid, smem);
+            } else {
+                if constexpr (cb_whole_job(l, false)) cb_run_job<l, false>(t, jobs, tid, smem);
+            }
+        });
+        return;
+    }
     if (t.kind == KIND_R2C) cb_dispatch_kind<KIND_R2C, -1>(t, jobs, tid, smem);
     else if (t.kind == KIND_C2R) cb_dispatch_kind<KIND_C2R, 1>(t, jobs, tid, smem);
     else if (t.dir < 0) cb_dispatch_kind<KIND_C2C, -1>(t, jobs, tid, smem);
@@ -183,7 +339,7 @@ __global__ void __launch_bounds__(CB_WG) conv_batch_kernel(CBArgs a) {
         // XCD's L2) before thread 0 publishes the task at the next iteration.
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
         __syncthreads();
-        prev_group = t.type == CB_INV ? -1 : t.group;
+        prev_group = t.type == CB_INV || t.type == CB_JOB ? -1 : t.group;
         finished_one = true;
     }
     // The last workgroup out clears the queue and readiness counters for the

@@ -78,13 +78,16 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         if (jobs[x].N != jobs[y].N) return jobs[x].N > jobs[y].N;
         return jobs[x].method < jobs[y].method;
     });
-    // Spectra: mono (N/2 + 1) bins each; stereo N bins each.
+    // Spectra of the jobs that run in parts: mono (N/2 + 1) bins each; stereo N
+    // bins each.
+    auto job_logn = [](unsigned N, bool stereo) { return ilog2(N) - (stereo ? 0 : 1); };
     std::vector<size_t> spec_off(count);
     size_t spec_points = 0;
     for (unsigned r = 0; r < count; ++r) {
         const mufft_hip_conv_job &j = jobs[order[r]];
         const bool stereo = (j.method & 1) == MUFFT_CONV_METHOD_FLAG_STEREO_MONO;
         spec_off[r] = spec_points;
+        if (cb_whole_job(job_logn(j.N, stereo), stereo)) continue;
         const size_t n = stereo ? j.N : j.N / 2 + 1;
         spec_points += 2 * ((n + 7) & ~(size_t)7);
     }
@@ -100,8 +103,11 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         CBJob &d = b->jobs[r];
         d.first = static_cast<const float2 *>(j.first);
         d.second = static_cast<const float2 *>(j.second);
-        d.spec1 = b->d_spectra.f2() + spec_off[r];
-        d.spec2 = d.spec1 + ((n + 7) & ~(size_t)7);
+        d.spec1 = d.spec2 = nullptr;
+        if (!cb_whole_job(job_logn(j.N, stereo), stereo)) {
+            d.spec1 = b->d_spectra.f2() + spec_off[r];
+            d.spec2 = d.spec1 + ((n + 7) & ~(size_t)7);
+        }
         d.out = static_cast<float2 *>(j.output);
     }
     // Twiddle tables per (log2 n, kind, direction) of the persistent kernel's variants.
@@ -140,12 +146,43 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         *stw = k.stw;
         return 0;
     };
+    // Every XCD needs workgroups of its own: launch all the resident ones
+    // (the dispatcher deals workgroups to the XCDs in turn).
+    const int resident = cb_resident_workgroups();
+    if (resident < CB_XCDS) {
+        set_err("occupancy query of the batch kernel failed");
+        destroy_batch(b);
+        return nullptr;
+    }
+    b->grid = resident / CB_XCDS * CB_XCDS;
+    // Whole jobs per task: a workgroup's capacity, less where the batch then
+    // makes fewer tasks than there are workgroups (each slot's work is its own
+    // from one wave per job group on, so emptier tasks end earlier).
+    auto jobs_per_task = [&](int logn, int div) {
+        const int cap = cb_jobs_per_task(logn), wave = cap * 64 / CB_WG;
+        return wave < 1 ? cap : std::max(wave, cap / div);
+    };
+    int job_div = 1;
+    for (; job_div < CB_WG / 64; job_div *= 2) {
+        size_t n = 0;
+        for (unsigned r = 0; r < count;) {
+            const mufft_hip_conv_job &j0 = jobs[order[r]];
+            unsigned e = r;
+            while (e < count && jobs[order[e]].N == j0.N && jobs[order[e]].method == j0.method) ++e;
+            const bool stereo = (j0.method & 1) == MUFFT_CONV_METHOD_FLAG_STEREO_MONO;
+            const int l = job_logn(j0.N, stereo);
+            const unsigned cap = cb_whole_job(l, stereo) ? (unsigned)jobs_per_task(l, job_div) : 1u;
+            n += (e - r + cap - 1) / cap;
+            r = e;
+        }
+        if (n >= (size_t)b->grid) break;
+    }
     // Job groups: runs of equal (N, method) jobs, chunked by the largest
     // workgroup capacity of the three transforms; each transform of a group
     // runs as tasks of its own capacity (two halves each at 2^CB_SPLIT_LOG2
     // points).  The group's inverse tasks wait for all its forward tasks.
     struct Group {
-        std::vector<CBTask> fwd, inv;
+        std::vector<CBTask> fwd, inv, whole;
         double cost = 0;
     };
     std::vector<Group> groups;
@@ -156,6 +193,37 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         unsigned e = r;
         while (e < count && jobs[order[e]].N == j0.N && jobs[order[e]].method == m0) ++e;
         const int lN = ilog2(j0.N);
+        const int lj = job_logn(j0.N, stereo);
+        if (cb_whole_job(lj, stereo)) {
+            float2 *tw = nullptr, *rtw = nullptr, *stw = nullptr, *twi = nullptr, *no = nullptr;
+            if (table_for(lj, stereo ? KIND_C2C : KIND_R2C, -1, &tw, &rtw, &stw) ||
+                table_for(lj, KIND_C2C, 1, &twi, &no, &no)) {
+                destroy_batch(b);
+                return nullptr;
+            }
+            const unsigned cap = (unsigned)jobs_per_task(lj, job_div);
+            for (unsigned q = r; q < e; q += cap) {
+                Group g;
+                CBTask t{};
+                t.type = CB_JOB;
+                t.kind = stereo ? KIND_C2C : KIND_R2C;
+                t.logn = lj;
+                t.job0 = (int)q;
+                t.njobs = (int)std::min<unsigned>(cap, e - q);
+                t.flags = ((m0 & MUFFT_CONV_METHOD_FLAG_ZERO_PAD_UPPER_HALF_FIRST) ? 1u : 0u) |
+                          ((m0 & MUFFT_CONV_METHOD_FLAG_ZERO_PAD_UPPER_HALF_SECOND) ? 2u : 0u);
+                t.norm = 1.0f / (float)j0.N;
+                t.tw = tw;
+                t.tw_inv = twi;
+                t.rtw = rtw;
+                t.group = (int)groups.size();
+                g.cost = 3.0 * t.njobs * (double)(1 << lj) * std::max(lj, 4);
+                g.whole.push_back(t);
+                groups.push_back(std::move(g));
+            }
+            r = e;
+            continue;
+        }
         struct Shape {
             int type, kind, dir, logn;
             unsigned flags;
@@ -218,7 +286,8 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         r = e;
     }
     // Groups to XCDs, longest first onto the least loaded; within an XCD the
-    // forward tasks longest first, then the inverse tasks in the same order.
+    // forward parts longest first, then the whole jobs in that order (the
+    // longest tasks, while the forward parts finish), then the inverse parts.
     std::vector<int> gorder(groups.size());
     for (size_t i = 0; i < groups.size(); ++i) gorder[i] = (int)i;
     std::stable_sort(gorder.begin(), gorder.end(),
@@ -238,20 +307,13 @@ static mufft_hip_conv_batch *mufft_hip_create_conv_batch_impl(const mufft_hip_co
         for (int gi : gorder)
             if (gx[gi] == xx) b->tasks.insert(b->tasks.end(), groups[gi].fwd.begin(), groups[gi].fwd.end());
         for (int gi : gorder)
+            if (gx[gi] == xx) b->tasks.insert(b->tasks.end(), groups[gi].whole.begin(), groups[gi].whole.end());
+        for (int gi : gorder)
             if (gx[gi] == xx) b->tasks.insert(b->tasks.end(), groups[gi].inv.begin(), groups[gi].inv.end());
     }
     a.qbegin[CB_XCDS] = (int)b->tasks.size();
     a.ngroups = (int)groups.size();
 
-    // Every XCD needs workgroups of its own: launch all the resident ones
-    // (the dispatcher deals workgroups to the XCDs in turn).
-    const int resident = cb_resident_workgroups();
-    if (resident < CB_XCDS) {
-        set_err("occupancy query of the batch kernel failed");
-        destroy_batch(b);
-        return nullptr;
-    }
-    b->grid = resident / CB_XCDS * CB_XCDS;
     // head[CB_XCDS] | ready[ngroups] as unsigned; finish, done, timeouts as 64-bit
     const size_t n32 = (size_t)CB_XCDS + groups.size();
     const size_t off64 = (n32 * sizeof(unsigned) + 7) & ~(size_t)7;

@@ -104,3 +104,34 @@ def test_batch_rejects_bad_jobs(gpu):
     for bad in ((6, MONO), (4, MONO), (131072, MONO), (65536, STEREO)):
         with pytest.raises(M.MufftError):
             M.ConvBatch([(bad[0], bad[1], x, x, x)])
+
+
+@pytest.mark.parametrize("pad", [0, 4, 8, 12])
+@pytest.mark.parametrize("count", [1, 5, 130])
+def test_whole_jobs_every_padding(gpu, pad, count):
+    """Jobs that run whole in one task: every size, the padding of each input,
+    partly filled tasks; against the FP64 circular convolution."""
+    import mufft_amd as M
+    import torch
+    rng = np.random.default_rng(100 + pad + count)
+    sizes = [(N, False) for N in (8, 16, 64, 128, 512, 2048, 4096)] + [(N, True) for N in (8, 32, 512, 1024, 2048, 16384)]
+    jobs, refs = [], []
+    for N, stereo in sizes:
+        for _ in range(count if N <= 512 else min(count, 3)):
+            na, nh = (N // 2 if pad & 4 else N), (N // 2 if pad & 8 else N)
+            a = rng.uniform(-1, 1, na).astype(np.float32)
+            if stereo:
+                a = (a + 1j * rng.uniform(-1, 1, na)).astype(np.complex64)
+            h = rng.standard_normal(nh).astype(np.float32)
+            out = torch.full((N,), 3.0, dtype=torch.complex64 if stereo else torch.float32, device=gpu)
+            jobs.append((N, (1 if stereo else 0) | pad, to_dev(a, gpu), to_dev(h, gpu), out))
+            y = np.fft.ifft(np.fft.fft(a.astype(np.complex128), N) * np.fft.fft(h.astype(np.complex128), N))
+            refs.append(y if stereo else y.real)
+    print(f"conv batch: padding {pad}, {len(jobs)} jobs", flush=True)
+    torch.cuda.synchronize()
+    b = M.ConvBatch(jobs)
+    for _ in range(2):
+        b.execute()
+        assert b.status() == 0
+    for j, ref in zip(jobs, refs):
+        assert rel_rms(from_dev(j[4]), ref) < 2e-6, (j[0], j[1])
