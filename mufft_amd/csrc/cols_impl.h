@@ -68,14 +68,19 @@ __global__ void __launch_bounds__(col_T(L_) * (TXP ? TXP : col_TX(L_)), col_wave
     // which spaces the loads out (2D c2c 4096^2 x 2 244 -> 222 us, c2r
     // 512^2 x 32 44.5 -> 41.2 us).
     constexpr bool ROW_ADDR = MODE != COL_PLAIN || L_ == 1024;
-    // Streaming only where a tile's row segments are whole 128-byte lines.
-    constexpr bool NT = MODE == COL_STREAM && TX >= 16;
+    // Streaming only where a tile's row segments are whole 128-byte lines.  The
+    // last of three launches streams too: c2c 2^24 x 2 303 -> 281 us, 2^23 x 8
+    // 630 -> 600, 2^26 663 -> 642; the middle one in place does not (2^24 x 2
+    // 282 -> 318).
+    constexpr bool NT = (MODE == COL_STREAM || MODE == COL_TWO_LEVEL) && TX >= 16;
     float2 v[E];
     const unsigned vin = ((unsigned)t * (unsigned)a.in_rs + (unsigned)colr) * 8u;
     static_for<0, E>([&](auto C) {
         constexpr int c = decltype(C)::value;
         if constexpr (ROW_ADDR) v[c] = gload<NT>(a.in + ib + (long long)(T * c) * a.in_rs, vin);
-        else v[c] = active ? (a.in + ib + col)[(long long)(t + T * c) * a.in_rs] : make_float2(0.f, 0.f);
+        // (Long columns: with the clamped column, 2D c2c 4096^2 x 2 takes 310 us.)
+        else if constexpr (L_ >= 4096) v[c] = active ? (a.in + ib + col)[(long long)(t + T * c) * a.in_rs] : make_float2(0.f, 0.f);
+        else v[c] = (a.in + ib + colr)[(long long)(t + T * c) * a.in_rs];
     });
 
     // COL_TWIDDLE: the twiddle of point t + T*c of a column with factor b is
