@@ -285,9 +285,10 @@ int run_cols(const Engine &e, const float2 *src, long long rs_src, long long bs_
         // up to 512 points: 2D c2c 512^2 x 64 115 -> 88 us, 256^2 x 100 40.2 ->
         // 36.2, 64 x 128 x 700 37.5 -> 33.1.  Not at 1024 points (1024^2 x 16 88.8
         // -> 93.3) nor for r2c, whose rows end in a partial tile (512^2 x 32 29.4
-        // -> 31.5).
+        // -> 31.5), nor where its narrow tiles would be taken (512^2 x 4 13.0 -> 13.8).
         const bool stream = src == dst && rs_src == rs_dst && bs_src == bs_dst && ncols == rs_src && e.col_tx == 0 &&
-                            e.logn >= 6 && e.logn <= 9 && ncols % col_TX(e.n) == 0 && bs_src % 16 == 0 &&
+                            e.logn >= 6 && e.logn <= 9 && ncols % col_TX(e.n) == 0 &&
+                            !use_narrow(e.n, col_TX(e.n), ncols, batch) && bs_src % 16 == 0 &&
                             reinterpret_cast<uintptr_t>(src) % 128 == 0;
         if (stream) HIP_TRY(launch_cols(e.logn, e.direction, a, st, COL_STREAM));
         else HIP_TRY(launch_cols(e.logn, e.direction, a, st, COL_PLAIN, tx));

@@ -111,11 +111,12 @@ int kernel_ptrs(T **p, R... rest) {
 }
 
 // ---- twiddle tables (FP64 on the GPU, rounded once) ------------------------
+// at: memory of the caller's for it (null: allocated).
 int build_stockham_table(int n, int direction, const std::vector<int> &radix, float2 **out,
-                         hipStream_t s);
+                         hipStream_t s, float2 *at = nullptr);
 int build_resolve_table(int n, int direction, float2 **out, hipStream_t s);
-// exp(dir * 2 pi i * j / n) for j < count.
-int build_plain_table(int n, int count, int direction, float2 **out, hipStream_t s);
+// exp(dir * 2 pi i * j / n) for j < count; spare: entries allocated behind it.
+int build_plain_table(int n, int count, int direction, float2 **out, hipStream_t s, int spare = 0);
 // Twiddles of a transform of n points split into n / n2 sub-transforms:
 // entry (k1 - 1) * n2 + j = exp(dir * 2 pi i * j * k1 / n).
 int build_split_table(int n, int n2, int direction, float2 **out, hipStream_t s);
@@ -165,7 +166,7 @@ struct Engine {
     int log_a = 0, log_b = 0, log_s2 = 0;
     int fs_code = 0;              // the split in use (fs_code_*)
     int col_tx = 0;               // column tile width (0 = col_TX_for(n, columns, images))
-    float2 *tw_self = nullptr;    // self-paired columns of a real transform (real_cols.hip)
+    float2 *tw_self = nullptr;    // (behind tw_fine) self-paired columns of a real transform (real_cols.hip)
     float2 *tw_pa = nullptr, *tw_pb = nullptr, *tw_coarse2 = nullptr, *tw_fine2 = nullptr;
     std::vector<int> gen_radix;
 

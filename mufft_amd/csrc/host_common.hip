@@ -80,7 +80,7 @@ int kernel_ptr(const void *ptr, const void **out) {
 
 // ---- twiddle tables ----------------------------------------------------------
 int build_stockham_table(int n, int direction, const std::vector<int> &radix, float2 **out,
-                         hipStream_t s) {
+                         hipStream_t s, float2 *at) {
     *out = nullptr;
     if (radix.size() <= 1) return 0;
     if (radix.size() > 24) {
@@ -100,7 +100,8 @@ int build_stockham_table(int n, int direction, const std::vector<int> &radix, fl
     }
     a.n = n;
     a.count = n - radix[0];
-    HIP_TRY(hipMalloc(out, sizeof(float2) * (size_t)a.count));
+    if (at) *out = at;
+    else HIP_TRY(hipMalloc(out, sizeof(float2) * (size_t)a.count));
     a.out = *out;
     HIP_TRY(launch_twiddles(a, s));
     return 0;
@@ -118,13 +119,13 @@ int build_resolve_table(int n, int direction, float2 **out, hipStream_t s) {
     return 0;
 }
 
-int build_plain_table(int n, int count, int direction, float2 **out, hipStream_t s) {
+int build_plain_table(int n, int count, int direction, float2 **out, hipStream_t s, int spare) {
     TwiddleArgs a{};
     a.direction = direction;
     a.mode = 2;
     a.n = n;
     a.count = count;
-    HIP_TRY(hipMalloc(out, sizeof(float2) * (size_t)count));
+    HIP_TRY(hipMalloc(out, sizeof(float2) * ((size_t)count + spare)));
     a.out = *out;
     HIP_TRY(launch_twiddles(a, s));
     return 0;
@@ -254,12 +255,20 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         log_s = log_n2;
         const int n1 = 1 << log_n1, n2 = 1 << log_n2;
         if (build_stockham_table(n1, dir, fused_sequence(n1, fs_E(n1), false), &tw_fs1, s) ||
-            build_plain_table(n >> log_s, n >> log_s, dir, &tw_coarse, s) ||
-            build_plain_table(n, 1 << log_s, dir, &tw_fine, s))
+            build_plain_table(n >> log_s, n >> log_s, dir, &tw_coarse, s))
             return -1;
         if (f3) {
             log_a = (f3 >> 4) & 15;
             log_b = f3 & 15;
+        }
+        // The real transforms' self-paired columns (r2c in the last launch, c2r
+        // in the first): their table sits behind tw_fine.
+        const int ns = kind == KIND_R2C && r2c_in_cols() ? 1 << (f3 ? log_b : log_n2)
+                     : kind == KIND_C2R && c2r_in_cols() ? n1 : 0;
+        if (build_plain_table(n, 1 << log_s, dir, &tw_fine, s, ns) ||
+            (ns && build_stockham_table(ns, dir, fused_sequence(ns, rcs_E(ns), false), &tw_self, s, tw_fine + (1 << log_s))))
+            return -1;
+        if (f3) {
             log_s2 = log_n2 / 2;
             const int na = 1 << log_a, nb = 1 << log_b;
             if (build_stockham_table(na, dir, fused_sequence(na, col_E(na), false), &tw_pa, s) ||
@@ -270,10 +279,6 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
         } else if (build_stockham_table(n2, dir, fused_sequence(n2, col_E(n2), false), &tw_fs2, s)) {
             return -1;
         }
-        // The real transforms' self-paired columns: r2c in the last launch, c2r in the first.
-        const int ns = kind == KIND_R2C && r2c_in_cols() ? 1 << (f3 ? log_b : log_n2)
-                     : kind == KIND_C2R && c2r_in_cols() ? n1 : 0;
-        if (ns && build_stockham_table(ns, dir, fused_sequence(ns, rcs_E(ns), false), &tw_self, s)) return -1;
     }
     if ((rows && !row_fused() && !four_step()) || (cols && !col_fused())) {
         gen_radix = generic_sequence(n);
@@ -284,7 +289,7 @@ int Engine::init(int n_, int dir, int kind, bool rows, bool cols, hipStream_t s,
 
 void Engine::release() {
     for (float2 *t : {tw_row, tw_col, tw_gen, tw_split, tw_fs1, tw_fs2, tw_coarse, tw_fine, tw_pa, tw_pb,
-                      tw_coarse2, tw_fine2, tw_self})
+                      tw_coarse2, tw_fine2})
         if (t) (void)hipFree(t);
     tw_row = tw_col = tw_gen = tw_split = nullptr;
     tw_fs1 = tw_fs2 = tw_coarse = tw_fine = nullptr;

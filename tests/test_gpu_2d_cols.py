@@ -154,3 +154,43 @@ def test_c2c_1024_squared_batch_of_16(gpu):
         orc = R.execute_plan_2d(R.create_plan_2d_c2c(n, n, d), x[15])
         assert rel_rms(y[15], orc) <= rms_tol_vs_mufft(n * n)
         del dy
+
+
+@pytest.mark.parametrize("Ny,Nx,B,off", [
+    (64, 64, 40, 0), (128, 64, 5, 0), (256, 32, 600, 0), (512, 64, 40, 0), (512, 512, 9, 0),  # streamed
+    (64, 32, 5, 0), (512, 8, 3, 0), (512, 64, 3, 0),   # tiles not full, too few
+    (256, 64, 5, 2),                   # images off a line's start
+])
+@pytest.mark.parametrize("d", [-1, 1])
+def test_c2c_streamed_columns(gpu, Ny, Nx, B, off, d):
+    """The column pass of whole images in place: streamed where tiles are whole
+    lines, plain elsewhere; within the bound, and the same bits per image in a
+    batch, alone, and with an explicit tile width."""
+    import mufft_amd as M
+    import torch
+    from mufft_amd import api
+    _flush(f"c2c 2D {Nx}x{Ny} x {B} offset {off} dir={d}")
+    x = cplx(0x3107 + Nx + Ny, B * Nx * Ny, 0.5).reshape(B, Ny, Nx)
+    dx = to_dev(x, gpu)
+    p = M.Plan2D("c2c", Nx, Ny, d)
+
+    def run(plan, src, b):
+        buf = torch.full((off + b * Nx * Ny + 16,), 3.0 + 0j, dtype=torch.complex64, device=gpu)
+        out = buf[off: off + b * Nx * Ny].view(b, Ny, Nx)
+        plan.execute_batched(out, src, b)
+        torch.cuda.synchronize()
+        assert bool((buf[:off] == 3.0).all()) and bool((buf[off + b * Nx * Ny:] == 3.0).all())
+        return from_dev(out)
+
+    y = run(p, dx, B)
+    for g in sorted({0, B // 2, B - 1}):
+        assert np.max(np.abs(y[g] - fp64.c2c_2d(x[g: g + 1], d)[0])) < abs_tol(Nx * Ny), g
+        assert np.array_equal(run(p, dx[g: g + 1], 1)[0], y[g]), g
+    if Ny >= 128:
+        old = api.get_column_tile(Ny)
+        try:
+            api.set_column_tile(Ny, {128: 64, 256: 32, 512: 8}[Ny])
+            assert np.array_equal(run(M.Plan2D("c2c", Nx, Ny, d), dx, B), y)
+        finally:
+            api.set_column_tile(Ny, 0)
+        assert api.get_column_tile(Ny) == old
