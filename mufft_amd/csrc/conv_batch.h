@@ -12,11 +12,12 @@ constexpr int CB_LDS_BYTES = 139264;  // 1024 threads x 17 padded points x 8 byt
 constexpr int CB_MIN_LOG2 = 2;        // smallest fused transform inside the kernel (4 points)
 constexpr int CB_SPLIT_LOG2 = 15;     // 32768 points: two workgroups per transform
 // Jobs that run whole in one task, by the points of their transforms: mono ones
-// whose threads lie in one wave (no workgroup barrier; 57 jobs of 1024 reals
-// 43 -> 31 us), stereo ones up to what a workgroup holds (128 jobs of 16384
-// points 70 -> 65 us, 256 87 -> 75).  Larger mono jobs run as fast or faster in
-// parts: whole, the three resolves' exchanges and spills cost what the saved
-// spectra gain (57 jobs of 32768 reals 57 -> 76 us).
+// whose threads lie in one wave (no workgroup barrier; in parts against whole,
+// us: 57 jobs of 1024 reals 37 / 28, 57 of 2048 reals 34.5 / 28), stereo ones up
+// to what a workgroup holds (of 16384 points: 128 jobs 59 / 53, 512 132 / 103).
+// Larger mono jobs run as fast or faster in parts: whole, the three resolves'
+// exchanges and spills cost what the saved spectra gain (57 jobs of 4096 reals
+// 40 / 46).
 MUFFT_HD constexpr bool cb_whole_job(int logn, bool stereo) { return logn <= (stereo ? 14 : 10); }
 
 // CB_JOB: both forward transforms, the product and the inverse transform of

@@ -37,6 +37,57 @@ int cb_jobs_per_task(int logn) {
 
 int cb_points_per_thread(int logn) { return rv_E(cb_sub_n(logn), cb_variant(cb_sub_n(logn))); }
 
+// Tasks and jobs are read by scalar loads, through a uniform pointer in the
+// constant address space (the tables never change once a batch is made).  A
+// task copied to the stack for the called functions cost every lane a store
+// and a load of it, and its fields and the pointers that hang on them vector
+// registers.  With the saves below, us: 640 jobs of mixed sizes 123 -> 97, 57
+// of 32768 reals 57 -> 47, 128 of 65536 reals 102 -> 81, 256 stereo jobs of
+// 16384 points 75 -> 60.
+template <typename P>
+using CBConst = const __attribute__((address_space(4))) P *;
+template <typename P>
+__device__ __forceinline__ CBConst<P> cb_const(const P *p) {
+    const unsigned long long u = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+    return (CBConst<P>)(((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ CBTask cb_load_task(const CBTask *p) {
+    CBConst<CBTask> q = cb_const(p);
+    CBTask t;
+    t.type = q->type;
+    t.kind = q->kind;
+    t.dir = q->dir;
+    t.logn = q->logn;
+    t.job0 = q->job0;
+    t.njobs = q->njobs;
+    t.flags = q->flags;
+    t.norm = q->norm;
+    t.tw = q->tw;
+    t.tw_inv = q->tw_inv;
+    t.rtw = q->rtw;
+    t.k1 = q->k1;
+    t.stw = q->stw;
+    t.group = q->group;
+    t.nprod = q->nprod;
+    return t;
+}
+__device__ __forceinline__ CBJob cb_load_job(const CBJob *jobs, int i) {
+    CBConst<CBJob> q = cb_const(jobs) + i;
+    CBJob j;
+    j.first = q->first;
+    j.second = q->second;
+    j.spec1 = q->spec1;
+    j.spec2 = q->spec2;
+    j.out = q->out;
+    return j;
+}
+
+// The task functions keep no register of their caller's unless a call to them
+// may be a tail call: then they save and restore up to 44 per lane.
+#define CB_NOTAIL __attribute__((not_tail_called))
+
 // Jobs [t.job0, t.job0 + t.njobs) of a task, one fused transform each; FL:
 // the task's flags if fixed at compile time (RF_DYNAMIC: t.flags).
 template <int KIND, int DIR, int LOGN, unsigned FL>
@@ -48,9 +99,9 @@ __device__ __forceinline__ void cb_run_rows(const CBTask &t, const CBJob *__rest
     constexpr int LDSN = rv_lds_per(N, VAR);
     static_assert(cb_lds_bytes(N) <= CB_LDS_BYTES, "LDS budget of the persistent kernel");
     const int lt = tid & (T - 1);
-    const int sub = tid / T;
+    const int sub = T >= 64 ? __builtin_amdgcn_readfirstlane(tid / T) : tid / T;
     const bool active = sub < t.njobs;
-    const CBJob &j = jobs[t.job0 + (active ? sub : 0)];
+    const CBJob j = cb_load_job(jobs, t.job0 + (active ? sub : 0));
     const float2 *X;
     const float2 *Y = nullptr;
     float2 *Xo;
@@ -76,7 +127,7 @@ __device__ __forceinline__ void cb_run_split(const CBTask &t, const CBJob *__res
     constexpr int N2 = 1 << (LOGN - 1);
     constexpr int VAR = cb_variant(N2);
     static_assert(cb_lds_bytes(N2) <= CB_LDS_BYTES, "LDS budget of the persistent kernel");
-    const CBJob &j = jobs[t.job0];
+    const CBJob j = cb_load_job(jobs, t.job0);
     const float2 *X = t.type == CB_FWD_FIRST ? j.first : (t.type == CB_FWD_SECOND ? j.second : j.spec1);
     const float2 *Y = t.type == CB_INV ? j.spec2 : nullptr;
     float2 *Xo = t.type == CB_FWD_FIRST ? j.spec1 : (t.type == CB_FWD_SECOND ? j.spec2 : j.out);
@@ -96,8 +147,9 @@ __device__ __forceinline__ void cb_run_fl(const CBTask &t, const CBJob *__restri
 // other set reads them at run time.  Mono: r2c, r2c, c2r with the multiply;
 // stereo: c2c, full r2c, c2c with the multiply (conv_batch_host.hip).
 template <int KIND, int DIR, int LOGN>
-__device__ __noinline__ void cb_run(const CBTask &t, const CBJob *__restrict__ jobs, int tid,
+__device__ __noinline__ CB_NOTAIL void cb_run(const CBTask *tp, const CBJob *__restrict__ jobs, int tid,
                                     float2 *smem) {
+    const CBTask t = cb_load_task(tp);
     constexpr unsigned FWD = RF_ZERO_PAD | RF_KEEP_OUT;
     if constexpr (KIND == KIND_R2C) {
         if (t.flags == FWD) return cb_run_fl<KIND, DIR, LOGN, FWD>(t, jobs, tid, smem);
@@ -138,7 +190,8 @@ struct CBGlobal {
 // so the product needs no other point.  Mono: the resolves (kernel.c:36-82)
 // pair points k and N-k through LDS.
 template <int LOGN, bool STEREO>
-__device__ __noinline__ void cb_run_job(const CBTask &t, const CBJob *__restrict__ jobs, int tid, float2 *smem) {
+__device__ __noinline__ CB_NOTAIL void cb_run_job(const CBTask *tp, const CBJob *__restrict__ jobs, int tid, float2 *smem) {
+    const CBTask t = cb_load_task(tp);
     constexpr int N = 1 << LOGN;
     constexpr int VAR = cb_variant(N);
     constexpr int E = rv_E(N, VAR);
@@ -152,7 +205,7 @@ __device__ __noinline__ void cb_run_job(const CBTask &t, const CBJob *__restrict
     const int sub = BUF ? __builtin_amdgcn_readfirstlane(tid / T) : tid / T;
     const bool active = sub < t.njobs;
     if (WAVE && !active) return;   // no barrier of the workgroup inside
-    const CBJob &j = jobs[t.job0 + (active ? sub : 0)];
+    const CBJob j = cb_load_job(jobs, t.job0 + (active ? sub : 0));
     float2 *L = smem + sub * rv_lds_per(N, VAR);
     auto slot = [](int o) { return pad_slot<LOGE>(o); };
     const bool zp1 = (t.flags & 1u) != 0, zp2 = (t.flags & 2u) != 0;
@@ -255,7 +308,7 @@ __device__ __noinline__ void cb_run_job(const CBTask &t, const CBJob *__restrict
 }
 
 template <int KIND_, int DIR_>
-__device__ __forceinline__ void cb_dispatch_kind(const CBTask &t, const CBJob *jobs, int tid, float2 *smem) {
+__device__ __forceinline__ void cb_dispatch_kind(const CBTask *tp, int logn, const CBJob *jobs, int tid, float2 *smem) {
     static_for<CB_MIN_LOG2, CB_SPLIT_LOG2 + 1>([&](auto L) {
         constexpr int l = decltype(L)::value;
         // Parts of the jobs that do not run whole: mono ones of l points, or
@@ -263,27 +316,27 @@ __device__ __forceinline__ void cb_dispatch_kind(const CBTask &t, const CBJob *j
         constexpr bool used = KIND_ == KIND_C2C ? !cb_whole_job(l, true)
                                                 : !cb_whole_job(l, false) || (KIND_ == KIND_R2C && !cb_whole_job(l + 1, true));
         if constexpr (used)
-            if (t.logn == l) cb_run<KIND_, DIR_, l>(t, jobs, tid, smem);
+            if (logn == l) cb_run<KIND_, DIR_, l>(tp, jobs, tid, smem);
     });
 }
 
-__device__ __forceinline__ void cb_run_task(const CBTask &t, const CBJob *jobs, int tid, float2 *smem) {
+__device__ __forceinline__ void cb_run_task(const CBTask *tp, const CBTask &t, const CBJob *jobs, int tid, float2 *smem) {
     if (t.type == CB_JOB) {
         static_for<CB_MIN_LOG2, CB_SPLIT_LOG2>([&](auto L) {
             constexpr int l = decltype(L)::value;
             if (t.logn != l) return;
             if (t.kind == KIND_C2C) {
-                if constexpr (cb_whole_job(l, true)) cb_run_job<l, true>(t, jobs, tid, smem);
+                if constexpr (cb_whole_job(l, true)) cb_run_job<l, true>(tp, jobs, tid, smem);
             } else {
-                if constexpr (cb_whole_job(l, false)) cb_run_job<l, false>(t, jobs, tid, smem);
+                if constexpr (cb_whole_job(l, false)) cb_run_job<l, false>(tp, jobs, tid, smem);
             }
         });
         return;
     }
-    if (t.kind == KIND_R2C) cb_dispatch_kind<KIND_R2C, -1>(t, jobs, tid, smem);
-    else if (t.kind == KIND_C2R) cb_dispatch_kind<KIND_C2R, 1>(t, jobs, tid, smem);
-    else if (t.dir < 0) cb_dispatch_kind<KIND_C2C, -1>(t, jobs, tid, smem);
-    else cb_dispatch_kind<KIND_C2C, 1>(t, jobs, tid, smem);
+    if (t.kind == KIND_R2C) cb_dispatch_kind<KIND_R2C, -1>(tp, t.logn, jobs, tid, smem);
+    else if (t.kind == KIND_C2R) cb_dispatch_kind<KIND_C2R, 1>(tp, t.logn, jobs, tid, smem);
+    else if (t.dir < 0) cb_dispatch_kind<KIND_C2C, -1>(tp, t.logn, jobs, tid, smem);
+    else cb_dispatch_kind<KIND_C2C, 1>(tp, t.logn, jobs, tid, smem);
 }
 
 // XCD (die) this workgroup runs on: the hardware XCC_ID register, bits 3:0.
@@ -333,8 +386,8 @@ __global__ void __launch_bounds__(CB_WG) conv_batch_kernel(CBArgs a) {
         const int local = __builtin_amdgcn_readfirstlane(s_local);
         __syncthreads();
         if (local >= qn) break;
-        const CBTask t = a.tasks[qb + local];
-        cb_run_task(t, a.jobs, tid, smem);
+        const CBTask t = cb_load_task(a.tasks + qb + local);
+        cb_run_task(a.tasks + qb + local, t, a.jobs, tid, smem);
         // Forward task: every thread's spectrum stores are complete (in this
         // XCD's L2) before thread 0 publishes the task at the next iteration.
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
